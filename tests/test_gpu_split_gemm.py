@@ -1,0 +1,173 @@
+"""The three-piece bf16 GEMMs (zk_split_*): tile edges, K tails, split-K, rows
+that are not float4-aligned, gathered rows, and operands that the pieces do not
+hold (infinities, values near the largest float, tiny ones), against float64
+and against the fp32 kernels (ZL_SPLIT_GEMM=0, read at zl_init)."""
+
+import os
+
+import numpy as np
+import pytest
+
+from zealot_amd import ops, synth
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def fp32_ctx():
+    from zealot_amd import Context
+
+    os.environ["ZL_SPLIT_GEMM"] = "0"
+    try:
+        c = Context(0)
+    finally:
+        del os.environ["ZL_SPLIT_GEMM"]
+    yield c
+    c.close()
+
+
+def product(ctx, L, R, lt, rt):
+    m, k, n = L.shape[0], L.shape[1], R.shape[1]
+    out = ctx.alloc((m, n))
+    dl = ctx.to_device(np.ascontiguousarray(L.T if lt else L))
+    dr = ctx.to_device(np.ascontiguousarray(R.T if rt else R))
+    ops.gemm(ctx, out, dl, lt, dr, rt, m, n, k)
+    return out.numpy()
+
+
+def used(ctx, fn):
+    """Names of the GEMM kernels that fn launches."""
+    import ctypes as C
+
+    ctx.check(ctx.lib.zl_timing_begin(ctx.h, b"*"))
+    fn()
+    n = C.c_longlong()
+    ctx.check(ctx.lib.zl_timing_end(ctx.h, None, C.byref(n), None))
+    names = []
+    for i in range(n.value):
+        name = C.c_char_p()
+        ctx.check(ctx.lib.zl_timing_launch(ctx.h, i, C.byref(name), None, None, None))
+        names.append(name.value.decode())
+    return names
+
+
+# (m, n, k, lhs_t, rhs_t): whole tiles; one past and one short of a tile in each
+# extent; K tails of 1, 31 and one k-tile; K not a multiple of 4 (element
+# loads); deep K with slices whose last one holds the tail.
+CASES = [(12288, 128, 32, False, True), (12289, 127, 33, False, True), (8191, 257, 96, False, True),
+         (12300, 130, 1, False, True), (6200, 256, 123, False, True), (256, 300, 8193, False, True),
+         (250, 24577, 516, False, False), (384, 11000, 261, False, False), (255, 16500, 200, True, False),
+         (129, 513, 24577, True, False), (128, 256, 6144, True, False)]
+
+
+@pytest.mark.parametrize("case", CASES)
+def test_split_gemm_edges(ctx, fp32_ctx, case):
+    m, n, k, lt, rt = case
+    g = np.random.default_rng(m + 3 * n + 7 * k)
+    L, R = synth.normal(g, (m, k)), synth.normal(g, (k, n))
+    got = []
+    names = used(ctx, lambda: got.append(product(ctx, L, R, lt, rt)))
+    assert any(x.startswith("zk_split") for x in names), names
+    ref = L.astype(np.float64) @ R.astype(np.float64)
+    # Six products per 16 reduction indices enter the fp32 accumulator, each
+    # rounded to 2^-24 of a partial sum below |L| |R|; the split-K slices and
+    # the dropped terms (2^-26) add less than 40 more.
+    bound = (6 * (-(-k // 16)) + 40) * 2.0 ** -24 * (np.abs(L).astype(np.float64) @ np.abs(R).astype(np.float64))
+    assert np.all(np.abs(got[0] - ref) <= bound), case
+    e = [np.linalg.norm(x - ref) / np.linalg.norm(ref) for x in (got[0], product(fp32_ctx, L, R, lt, rt))]
+    print(f"[gpu] split gemm {case}: relative error {e[0]:.2e}, fp32 kernels {e[1]:.2e}", flush=True)
+
+
+@pytest.mark.parametrize("what", ["inf", "-inf", "nan", "max", "tiny", "zero"])
+@pytest.mark.parametrize("lt,rt", [(False, True), (False, False), (True, False)])
+def test_split_gemm_special_values(ctx, fp32_ctx, what, lt, rt):
+    """Infinities, NaN, values that round to a bf16 infinity and operands whose
+    low pieces leave the bf16 range give what the fp32 kernels give."""
+    m, n, k = 1100, 4200, 300
+    g = np.random.default_rng(5)
+    L, R = synth.normal(g, (m, k)), synth.normal(g, (k, n), 0.05)
+    if what == "tiny":
+        L = (L * np.float32(1e-36)).astype(np.float32)
+    elif what == "zero":
+        L[:] = 0.0
+    else:
+        v = {"inf": np.inf, "-inf": -np.inf, "nan": np.nan, "max": np.finfo(np.float32).max}[what]
+        L[700, 17] = v
+        R[17, :] = np.where(np.abs(R[17, :]) < 1e-3, 1e-3, R[17, :])
+    assert any(x.startswith("zk_split") for x in used(ctx, lambda: product(ctx, L, R, lt, rt)))
+    a, b = product(ctx, L, R, lt, rt), product(fp32_ctx, L, R, lt, rt)
+    assert np.array_equal(np.isnan(a), np.isnan(b))
+    inf = np.isinf(b)
+    assert np.array_equal(inf, np.isinf(a)) and np.array_equal(a[inf], b[inf])
+    ok = np.isfinite(b)
+    # Both sums lie within K roundings of 2^-24 of |L| |R|.
+    with np.errstate(invalid="ignore", over="ignore"):
+        bound = 2 * k * 2.0 ** -24 * (np.abs(L).astype(np.float64) @ np.abs(R).astype(np.float64))
+    d = np.abs(a[ok].astype(np.float64) - b[ok])
+    assert np.all(d <= np.maximum(bound[ok], 0.0) + 1e-45)
+
+
+@pytest.mark.parametrize("rows", [12288, 12301])
+def test_split_gemm_network(ctx, rows):
+    """Forward (both accumulator forms), data and weight gradients of a
+    network at whole and ragged row counts against float64."""
+    from zealot_amd.rl import GpuMlp, unpack
+
+    dims = [123, 512, 256, 128, 29]
+    g = np.random.default_rng(rows)
+    packed = synth.kaiming_uniform_net(g, dims, 0.1)
+    x, gout = synth.normal(g, (rows, 123)), synth.normal(g, (rows, 29))
+    mlp = GpuMlp(ctx, dims, rows + 100)
+    mlp.write_weights(packed)
+    dx, dg = ctx.to_device(x), ctx.to_device(gout)
+
+    def go():
+        mlp.forward(dx, rows)
+        mlp.backward(dg)
+
+    names = used(ctx, go)
+    assert {"zk_split_ak_bk_s", "zk_split_ak_bk_acc2", "zk_split_ak_bn_dg", "zk_split_am_bn"} <= set(names), names
+    ws, bs = unpack(dims, packed.astype(np.float64))
+    acts = [x.astype(np.float64)]
+    for i, (w, b) in enumerate(zip(ws, bs)):
+        z = acts[-1] @ w.T + b
+        acts.append(np.where(z > 0, z, np.expm1(np.minimum(z, 0))) if i < 3 else z)
+    d, parts = gout.astype(np.float64), []
+    for i in range(3, -1, -1):
+        parts = [(d.T @ acts[i]).ravel(), d.sum(0)] + parts
+        if i:
+            d = (d @ ws[i]) * np.where(acts[i] > 0, 1.0, acts[i] + 1.0)
+    out, grads = mlp.output(rows), mlp.read_grads()
+    assert np.max(np.abs(out - acts[-1])) <= 1e-5 * np.max(np.abs(acts[-1]))
+    o = 0
+    for p in parts:  # the bar of the gradient tests is 1e-4 of each tensor's largest value
+        assert np.max(np.abs(grads[o:o + p.size] - p)) <= 1e-5 * np.max(np.abs(p))
+        o += p.size
+    mlp.close()
+
+
+def test_split_gemm_gathered_rows(ctx):
+    """A shuffled minibatch of a ragged number of rows (the observation gather
+    inside the first layer's forward and weight gradient): the same rows in
+    another order, so the first Adam moments agree to the rounding of a sum."""
+    from zealot_amd.rl import DeviceBatch, GpuActorCritic, PpoConfig
+
+    ad, cd = [64, 512, 256, 128, 12], [64, 512, 256, 128, 1]
+    n = 13001
+    g = np.random.default_rng(9)
+    actor, critic = synth.kaiming_uniform_net(g, ad, 0.1), synth.kaiming_uniform_net(g, cd, 0.1)
+    obs = synth.obs(g, n, 64)
+    args = [obs, obs, synth.normal(g, (n, 12)), synth.normal(g, (n, 12)), synth.normal(g, n) - 20, synth.normal(g, n),
+            synth.normal(g, n), synth.normal(g, n)]
+    out = []
+    for shuffle in (True, False):
+        gac = GpuActorCritic(ctx, ad, cd, n)
+        gac.set_params(actor, critic, np.full(12, -0.5, np.float32), 1e-4)
+        db = DeviceBatch(ctx, *args)
+        gac.update(db, PpoConfig(epochs=1, minibatches=1, shuffle=shuffle, normalize_adv=False))
+        out.append(gac.get_moments())
+        gac.close()
+    for i in (0, 2, 4):
+        a, b = out[0][i], out[1][i]
+        assert np.any(b != 0)
+        assert np.max(np.abs(a - b)) <= 1e-5 * np.max(np.abs(b)), i

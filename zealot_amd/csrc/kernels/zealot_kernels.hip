@@ -3,6 +3,7 @@
 // name; see gemm_mfma.hip, narrow.hip, ppo_kernels.hip, head.hip and
 // obs_norm.hip.
 #include "gemm_mfma.hip"
+#include "gemm_split.hip"
 #include "narrow.hip"
 #include "obs_norm.hip"
 #include "ppo_kernels.hip"

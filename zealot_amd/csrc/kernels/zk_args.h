@@ -40,7 +40,8 @@ struct GemmArgs {
   int bias_stride;
   int epi;
   int act;                 // ELU in the bias epilogues
-  int vecA, vecB;          // float4 global loads are aligned and in bounds
+  int vecA, vecB;          // float4 global loads are aligned and in bounds (three-piece GEMMs: vecB =
+                           // C's and Y's rows are)
   int kt_per_split;        // k-tiles per split-K slice (narrow weight gradient: rows)
   int nsplit;              // split-K slices of this problem
 };

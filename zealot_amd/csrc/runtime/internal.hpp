@@ -49,6 +49,7 @@ enum KernelId : int {
   K_GEMM_BWD_64,
   K_GEMM_BWD_128_D128,
   K_GEMM_BWD_64_D128,
+  K_SPLIT_BWD,
   K_HEAD_FWD,
   K_HEAD_FWD_X,
   K_POLICY,
@@ -57,10 +58,12 @@ enum KernelId : int {
   K_GEMM_BASE
 };
 
-// Kernel family of a GEMM variant: LDS-tiled (gemm_mfma.hip) or one of the
+// Kernel family of a GEMM variant: LDS-tiled (gemm_mfma.hip), three-piece bf16
+// (gemm_split.hip, launched and split over K like the tiled ones) or one of the
 // register-resident narrow kernels (narrow.hip): N <= 32 (forward of an
 // output layer), K <= 32 (its data gradient), M <= 32 (its weight gradient).
-enum GemmKind : int { G_TILED = 0, G_NARROW_N = 1, G_NARROW_K = 2, G_NARROW_M = 3 };
+enum GemmKind : int { G_TILED = 0, G_NARROW_N = 1, G_NARROW_K = 2, G_NARROW_M = 3, G_SPLIT = 4 };
+inline bool is_tiled(int kind) { return kind == G_TILED || kind == G_SPLIT; }
 
 // One GEMM variant: operand orientation, tile (for the narrow kernels: rows
 // per block and the largest narrow dimension), k-tile, block size, whether it
@@ -153,6 +156,9 @@ struct zl_ctx {
   // layout (ZL_GEMM_AKBK / _AKBN / _AMBN / _AMBK), split-K slice count
   // (ZL_SPLITK) and the split-K target grid size (ZL_SPLITK_TARGET).
   int force_gemm[4] = {-1, -1, -1, -1};
+  // Three-piece bf16 GEMMs where pick_gemm's rule takes them (ZL_SPLIT_GEMM=0
+  // turns them off).
+  bool split_gemm = true;
   int force_splits = 0;
   int splitk_target = 256;
   // Divisor of the split-K slice count of weight gradients that share a
@@ -252,10 +258,14 @@ struct GemmDesc {
 // vec: both operands can be read as aligned float4 rows (see run_gemm).
 // vec_b: B alone can be read as float4 rows and the problem has no split-K,
 // row sums or gathers (the small-K variants may then take it).
+// kvec: every K-contiguous operand can be read as float4 rows (the three-piece
+// variants read the others by elements).
 int pick_gemm(const zl_ctx* c, int M, int N, int K, bool a_kc, bool b_kc, bool vec = true,
-              int epi = zk::kEpiStore, bool vec_b = false);
+              int epi = zk::kEpiStore, bool vec_b = false, bool kvec = true);
 int gemm_splits(const zl_ctx* c, int M, int N, int K, bool a_kc, bool b_kc, int epi,
                 bool vec = true);
+// Whether a row-major forward layer takes the three-piece bf16 kernels.
+bool split_forward(const zl_ctx* c, int M, int N, int K);
 size_t gemm_ws_floats(const zl_ctx* c, int M, int N, int K, bool a_kc, bool b_kc, int epi);
 zl_status run_gemm(zl_ctx* c, const GemmDesc& d);
 // One launch for n (1 or 2) problems that pick the same variant (else n

@@ -899,6 +899,8 @@ zl_status minibatch_pass(zl_ppo* p, const NetView v[2], const int* px, const int
     hfwd = ((uintptr_t)nb.act[l] & 15) == 0 && ((uintptr_t)w2 & 15) == 0 && nb.ld[l] % 4 == 0 &&
            nl.ldw[l] % 4 == 0;
     hfwd_exact = hfwd_exact && nl.dims[l + 1] == zk::kHeadMaxHidden && nl.dims[l] % 32 == 0;
+    // A layer that the three-piece kernels take is faster as its own launch.
+    hfwd = hfwd && !split_forward(c, rows, nl.dims[l + 1], nl.dims[l]);
   }
   zl_status s = pair_forward(c, v, p->params, px, rows, guard,
                              p->fused_head ? (hfwd ? La - 2 : La - 1) : -1);

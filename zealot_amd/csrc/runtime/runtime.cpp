@@ -23,7 +23,7 @@ const char* const kFixedNames[K_GEMM_BASE] = {
     "zk_norm_apply",
     "zk_norm_stats",    "zk_norm_merge",  "zk_norm_commit", "zk_sample_g32",  "zk_sample_g64",
     "zk_stage",         "zk_sumsq_multi", "zk_clip_scale",  "zk_adam_multi",
-    "zk_gemm_bwd_128x128_dg_x", "zk_gemm_bwd_64x128_dg_x", "zk_gemm_bwd_128x128_dg128_x", "zk_gemm_bwd_64x128_dg128_x", "zk_head_fwd", "zk_head_fwd_x",
+    "zk_gemm_bwd_128x128_dg_x", "zk_gemm_bwd_64x128_dg_x", "zk_gemm_bwd_128x128_dg128_x", "zk_gemm_bwd_64x128_dg128_x", "zk_split_bwd", "zk_head_fwd", "zk_head_fwd_x",
     "zk_policy",        "zk_transpose",   "zk_policy_pack",
 };
 
@@ -62,6 +62,13 @@ const GemmKernel kGemmTable[] = {
     {"zk_gemm_ak_bn_64x64xk128_w22", true, false, 64, 64, 128, 256, true},
     {"zk_gemm_ak_bn_64x64xk128_w24_s", true, false, 64, 64, 128, 512, false, G_TILED, true},
     {"zk_gemm_ak_bn_64x64xk128_w24", true, false, 64, 64, 128, 512, true},
+    {"zk_split_ak_bk", true, true, 128, 128, 32, 256, true, G_SPLIT},
+    {"zk_split_ak_bk_acc2", true, true, 128, 128, 32, 256, true, G_SPLIT},
+    {"zk_split_ak_bk_s", true, true, 128, 128, 32, 256, false, G_SPLIT},
+    {"zk_split_ak_bn", true, false, 128, 128, 32, 256, true, G_SPLIT},
+    {"zk_split_ak_bn_s", true, false, 128, 128, 32, 256, false, G_SPLIT},
+    {"zk_split_ak_bn_dg", true, false, 128, 128, 32, 256, true, G_SPLIT},
+    {"zk_split_am_bn", false, false, 128, 128, 32, 256, false, G_SPLIT},
     {"zk_narrow_n1_v", true, true, kNarrowRows, 16, 16, 256, true, G_NARROW_N},
     {"zk_narrow_n2_v", true, true, kNarrowRows, 32, 16, 256, true, G_NARROW_N},
     {"zk_narrow_n1_s", true, true, kNarrowRows, 16, 16, 256, false, G_NARROW_N},
@@ -162,8 +169,59 @@ static bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
 // 512- and 256-wide layers, 64 x 128 for the 128-wide one (both with 32-row
 // k-tiles, so that the k-loop's barrier sits between two chunks) and
 // 32 x 128 for the narrow heads (measured on gfx950 at 24,576 rows).
+// The three-piece bf16 variant (gemm_split.hip) of a product, or -1 where the
+// fp32 tiles stay. Its 128 x 128 tiles pay once enough of them are in flight;
+// fewer are bound by one block's serial chain (2 us per k-tile), which the
+// smaller fp32 tiles shorten. Launches of an actor + critic pair, us, fp32 vs
+// three-piece: forward 2,000 x 512 x 128 13 / 16, 3,000 x 256 x 512 29 / 34,
+// 4,500 x 256 x 512 37 / 33, 24,576 x 256 x 512 108 / 79, 24,576 x 512 x 128
+// 70 / 49; a layer's backward 1,000 x 512 x 256 43 / 28 + 26, 2,000 51 / 33,
+// 24,576 222 / 151; input-layer weight gradient 512 x 128 x 24,576 63 / 48.
+// Feature-major products (L_AK_BN without ELU'), one problem: 128 x 24,576 x
+// 256 26 / 29, 256 x 24,576 x 512 75 / 60. Narrow or half-empty tiles keep fp32.
+static int pick_split(const zl_ctx* c, int M, int N, int K, int lay, int epi, bool kvec) {
+  if (!c || !c->split_gemm || lay == L_AM_BK) return -1;
+  const long long tiles = cdiv(M, 128) * cdiv(N, 128);
+  if (2LL * M * N < tiles * 128 * 128) return -1;
+  // Split-K slices of at least eight k-tiles count as blocks.
+  const long long slices = epi == zk::kEpiStore ? std::max<long long>(1, std::min<long long>(cdiv(256, tiles), K / 256)) : 1;
+  long long least = 48;
+  if (lay == L_AK_BK && epi != zk::kEpiStore) least = M > 2048 ? 64 : LLONG_MAX;
+  if (lay == L_AK_BN && epi != zk::kEpiEluGrad) least = 256;
+  if (tiles * slices < least) return -1;
+  switch (lay) {
+    case L_AK_BK:
+      if (!kvec) return gemm_id("zk_split_ak_bk_s");
+      return gemm_id(epi != zk::kEpiStore && K > 128 ? "zk_split_ak_bk_acc2" : "zk_split_ak_bk");
+    case L_AK_BN:
+      if (!kvec) return gemm_id("zk_split_ak_bn_s");
+      return gemm_id(epi == zk::kEpiEluGrad ? "zk_split_ak_bn_dg" : "zk_split_ak_bn");
+    default:
+      return gemm_id("zk_split_am_bn");
+  }
+}
+
+bool split_forward(const zl_ctx* c, int M, int N, int K) {
+  return c->force_gemm[L_AK_BK] < 0 && pick_split(c, M, N, K, L_AK_BK, zk::kEpiBiasN, true) >= 0;
+}
+
+static int pick_fp32(const zl_ctx* c, int M, int N, int K, bool a_kc, bool b_kc, bool vec, int epi,
+                     bool vec_b);
+
 int pick_gemm(const zl_ctx* c, int M, int N, int K, bool a_kc, bool b_kc, bool vec, int epi,
-              bool vec_b) {
+              bool vec_b, bool kvec) {
+  const int fp32 = pick_fp32(c, M, N, K, a_kc, b_kc, vec, epi, vec_b);
+  const int lay = layout_of(a_kc, b_kc);
+  if ((c && c->force_gemm[lay] >= 0) || fp32 < 0) return fp32;
+  // Narrow and small-K shapes keep their own kernels.
+  const GemmKernel& g = kGemmTable[fp32 - K_GEMM_BASE];
+  if (g.kind != G_TILED || strstr(g.name, "xk128")) return fp32;
+  const int split = pick_split(c, M, N, K, lay, epi, kvec);
+  return split >= 0 ? split : fp32;
+}
+
+static int pick_fp32(const zl_ctx* c, int M, int N, int K, bool a_kc, bool b_kc, bool vec, int epi,
+                     bool vec_b) {
   const int lay = layout_of(a_kc, b_kc);
   const bool forced = c && c->force_gemm[lay] >= 0;
   // K <= 128 with B float4-aligned: one round of loads for the whole K
@@ -274,7 +332,7 @@ static int narrow_rows_per_slice(const zl_ctx* c, int N, int K, int epi) {
 int gemm_splits(const zl_ctx* c, int M, int N, int K, bool a_kc, bool b_kc, int epi, bool vec) {
   const GemmKernel& g = kGemmTable[pick_gemm(c, M, N, K, a_kc, b_kc, vec) - K_GEMM_BASE];
   if (g.kind == G_NARROW_M) return (int)cdiv(std::max(K, 1), narrow_rows_per_slice(c, N, K, epi));
-  if (g.kind != G_TILED) return 1;
+  if (!is_tiled(g.kind)) return 1;
   if (epi != zk::kEpiStore) return 1;
   const long long tiles = cdiv(M, g.bm) * cdiv(N, g.bn);
   const long long kt = cdiv(K, g.bk);
@@ -301,12 +359,33 @@ int gemm_splits(const zl_ctx* c, int M, int N, int K, bool a_kc, bool b_kc, int 
   return (int)cdiv(kt, per);
 }
 
+// An upper bound of the split-K scratch over every batch of up to K rows: the
+// slice count is not monotonic in K (slices are whole k-tiles), and a smaller
+// K can take another variant, so each variant's slice limit counts.
 size_t gemm_ws_floats(const zl_ctx* c, int M, int N, int K, bool a_kc, bool b_kc, int epi) {
-  // Enough for either variant family (operand alignment is known at launch).
-  int s = std::max(gemm_splits(c, M, N, K, a_kc, b_kc, epi, true),
-                   gemm_splits(c, M, N, K, a_kc, b_kc, epi, false));
-  if (s <= 1) return 0;
-  return (size_t)s * M * N + (size_t)s * M;
+  if (epi != zk::kEpiStore) return 0;
+  long long s = 1;
+  const int lay = layout_of(a_kc, b_kc);
+  auto limit = [&](int kid) {
+    const GemmKernel& g = kGemmTable[kid - K_GEMM_BASE];
+    if (g.kind == G_NARROW_M) {
+      const long long gy = cdiv(N, kNarrowCols);
+      s = std::max(s, std::min<long long>(std::max<long long>(1, (c ? c->narrow_target : 256) / gy),
+                                          cdiv(std::max(K, 1), kNarrowSliceQuantum)));
+    } else if (is_tiled(g.kind)) {
+      const long long kt = cdiv(K, g.bk);
+      if (c && c->force_splits > 0) {
+        s = std::max<long long>(s, std::min<long long>(c->force_splits, std::max<long long>(1, kt)));
+        return;
+      }
+      const long long target = 2LL * (c ? c->splitk_target : 256);
+      s = std::max(s, std::min<long long>(cdiv(target, cdiv(M, g.bm) * cdiv(N, g.bn)), std::max<long long>(1, kt / 8)));
+    }
+  };
+  const int split = pick_split(c, M, N, K, lay, epi, true);
+  if (split >= 0) limit(split);
+  for (bool vec : {true, false}) limit(pick_fp32(c, M, N, K, a_kc, b_kc, vec, epi, false));
+  return s <= 1 ? 0 : (size_t)s * M * N + (size_t)s * M;
 }
 
 static int reduce_lanes(int splits);
@@ -324,6 +403,7 @@ zl_status launch_splitk_reduce(zl_ctx* c, zk::SplitReduceArgs& r) {
 struct GemmPlan {
   int kid = -1;
   bool vec = false;
+  bool vec_out = false;  // float4-aligned rows of C (and of the ELU' operand)
   int splits = 1, per = 0;
   unsigned gx = 0, gy = 0;
 };
@@ -336,11 +416,15 @@ static zl_status plan_gemm(zl_ctx* c, const GemmDesc& d, GemmPlan& P) {
   const bool vb = aligned16(d.B) && d.ldb % 4 == 0 && d.ldb >= round_up(b_ext, 4);
   P.vec = va && vb;
   const bool plain = !d.rowsum_out && !d.permA && !d.permB && d.splits <= 1;
-  P.kid = pick_gemm(c, d.M, d.N, d.K, d.a_kc, d.b_kc, P.vec, d.epi, vb && plain);
+  const bool kvec = (!d.a_kc || va) && (!d.b_kc || vb);
+  P.kid = pick_gemm(c, d.M, d.N, d.K, d.a_kc, d.b_kc, P.vec, d.epi, vb && plain, kvec);
   if (P.kid < 0) return fail(c, ZL_ERR_INVALID, "no GEMM variant for this layout");
   const GemmKernel& g = kGemmTable[P.kid - K_GEMM_BASE];
-  if (g.a_kc != d.a_kc || g.b_kc != d.b_kc || (g.vec && !P.vec) || (g.need_vec_b && !(vb && plain)))
+  const bool vec_ok = g.kind == G_SPLIT ? kvec : P.vec;
+  if (g.a_kc != d.a_kc || g.b_kc != d.b_kc || (g.vec && !vec_ok) || (g.need_vec_b && !(vb && plain)))
     return fail(c, ZL_ERR_INVALID, "GEMM variant %s does not match the operand layout", g.name);
+  if (g.kind == G_SPLIT && ((d.permA && !d.a_kc) || (d.permB && d.b_kc)))
+    return fail(c, ZL_ERR_INVALID, "GEMM variant %s gathers storage rows of A[M][K] and B[K][N] only", g.name);
   if (strstr(g.name, "xk128") && (d.K > 128 || !plain))
     return fail(c, ZL_ERR_INVALID, "GEMM variant %s takes K <= 128 without split-K, row sums or gathers",
                 g.name);
@@ -367,6 +451,7 @@ static zl_status plan_gemm(zl_ctx* c, const GemmDesc& d, GemmPlan& P) {
     // those rows must be 16-byte aligned, unless C is the split-K scratch).
     const bool c_vec = P.splits > 1 || (aligned16(d.C) && d.ldc % 4 == 0);
     const bool y_vec = d.epi != zk::kEpiEluGrad || (aligned16(d.Y) && d.ldy % 4 == 0);
+    P.vec_out = c_vec && y_vec;
     if (d.K > 0 && d.M % g.bm == 0 && d.N % g.bn == 0 && d.K % g.bk == 0 && c_vec && y_vec) {
       const int x = exact_form(P.kid);
       if (x >= 0) P.kid = x;
@@ -411,8 +496,8 @@ static zl_status plan_batch(zl_ctx* c, const GemmDesc* d, int n, BatchLaunch& L,
   // shape share such a launch. (Tiled kernels give each problem its own
   // block range, so the actor's and the critic's layer share a launch
   // whatever their shapes.)
-  const bool narrow_pair = nl == 2 && kGemmTable[P[0].kid - K_GEMM_BASE].kind != G_TILED &&
-                           kGemmTable[P[1].kid - K_GEMM_BASE].kind != G_TILED;
+  const bool narrow_pair = nl == 2 && !is_tiled(kGemmTable[P[0].kid - K_GEMM_BASE].kind) &&
+                           !is_tiled(kGemmTable[P[1].kid - K_GEMM_BASE].kind);
   if (narrow_pair &&
       (live[0]->M != live[1]->M || live[0]->N != live[1]->N || live[0]->K != live[1]->K))
     return ZL_OK;
@@ -420,6 +505,12 @@ static zl_status plan_batch(zl_ctx* c, const GemmDesc* d, int n, BatchLaunch& L,
   // the general form.
   if (nl == 2 && P[0].kid != P[1].kid && inexact_form(P[0].kid) == inexact_form(P[1].kid))
     P[0].kid = P[1].kid = inexact_form(P[0].kid);
+  // Two forwards of which one takes the two-accumulator form share it.
+  const int acc2 = gemm_id("zk_split_ak_bk_acc2");
+  if (nl == 2 && P[0].kid != P[1].kid && (P[0].kid == acc2 || P[1].kid == acc2)) {
+    const int other = P[0].kid == acc2 ? P[1].kid : P[0].kid;
+    if (other == gemm_id("zk_split_ak_bk") && P[0].splits == 1 && P[1].splits == 1) P[0].kid = P[1].kid = acc2;
+  }
   if (nl == 2 && P[0].kid != P[1].kid) {
     // Two narrow problems of one family that differ only in the template
     // width (16 vs 32 columns / rows, float4 vs element loads) share the
@@ -467,7 +558,7 @@ static zl_status plan_batch(zl_ctx* c, const GemmDesc* d, int n, BatchLaunch& L,
     a.kt_per_split = P[i].per;
     a.nsplit = P[i].splits;
     a.vecA = P[i].vec;
-    a.vecB = P[i].vec;
+    a.vecB = g.kind == G_SPLIT ? P[i].vec_out : P[i].vec;
     L.part[i] = nullptr;
     if (P[i].splits == 1) {
       a.C = q.C;
@@ -498,7 +589,7 @@ static zl_status plan_batch(zl_ctx* c, const GemmDesc* d, int n, BatchLaunch& L,
     flops += 2.0 * q.M * (q.N_alg > 0 ? q.N_alg : q.N) * (double)(q.K_alg > 0 ? q.K_alg : q.K);
   }
   L.kid = P[0].kid;
-  if (g.kind == G_TILED) {  // one block range per problem, a 1-D grid
+  if (is_tiled(g.kind)) {  // one block range per problem, a 1-D grid
     long long blk = 0;
     for (int i = 0; i < nl; ++i) {
       B.blk0[i] = (int)blk;
@@ -596,6 +687,12 @@ zl_status run_gemm_bwd(zl_ctx* c, const GemmDesc* w, int nw, const GemmDesc* d, 
       else if (W.kid == gemm_id("zk_gemm_am_bn_64x128x32_w24_x"))
         mk = K_GEMM_BWD_64_D128;
     }
+    unsigned threads = 512;
+    if (ow && od && W.nl > 0 && D.nl > 0 && D.kid == gemm_id("zk_split_ak_bn_dg") &&
+        W.kid == gemm_id("zk_split_am_bn")) {
+      mk = K_SPLIT_BWD;
+      threads = 256;
+    }
     if (mk >= 0) {
       zk::GemmPair a{};
       a.w = W.B;
@@ -604,7 +701,7 @@ zl_status run_gemm_bwd(zl_ctx* c, const GemmDesc* w, int nw, const GemmDesc* d, 
       const long long blocks = (long long)W.gx + D.gx;
       c->pending_flops = W.flops + D.flops;
       c->pending_shape = {D.live[0]->M, D.live[0]->N, D.live[0]->K, W.P[0].splits};
-      s = launch(c, mk, (unsigned)blocks, 1, 1, a, 0, 512);
+      s = launch(c, mk, (unsigned)blocks, 1, 1, a, 0, threads);
       if (!s) s = finish_batch(c, W);
       return s ? s : finish_batch(c, D);
     }
@@ -904,6 +1001,7 @@ zl_status zl_init(int device, zl_ctx** out) {
     }
     c->force_gemm[l] = id;
   }
+  if (const char* v = getenv("ZL_SPLIT_GEMM")) c->split_gemm = atoi(v) != 0;
   if (const char* v = getenv("ZL_SPLITK")) c->force_splits = std::max(0, atoi(v));
   if (const char* v = getenv("ZL_SPLITK_TARGET")) c->splitk_target = std::max(1, atoi(v));
   if (const char* v = getenv("ZL_BWD_SPLIT_DIV")) c->bwd_split_div = std::max(0, atoi(v));
