@@ -171,3 +171,18 @@ def test_split_gemm_gathered_rows(ctx):
         a, b = out[0][i], out[1][i]
         assert np.any(b != 0)
         assert np.max(np.abs(a - b)) <= 1e-5 * np.max(np.abs(b)), i
+
+
+# (m, n, k): weight gradients of short batches: no slice, one k-tile more than a
+# slice pair, the slice cap, one row past it; 64-, 96- and 128-wide tiles.
+@pytest.mark.parametrize("m,n,k", [(512, 128, 96), (512, 128, 129), (256, 288, 384), (512, 64, 385), (128, 256, 960),
+                                   (128, 128, 4096), (128, 128, 4097), (100, 124, 700)])
+def test_short_reductions_are_sliced(ctx, m, n, k):
+    g = np.random.default_rng(m + n + k)
+    L, R = synth.normal(g, (m, k)), synth.normal(g, (k, n))
+    got = []
+    used(ctx, lambda: got.append(product(ctx, L, R, True, False)))
+    ref = L.astype(np.float64) @ R.astype(np.float64)
+    bound = (6 * (-(-k // 16)) + 104) * 2.0 ** -24 * (np.abs(L).astype(np.float64) @ np.abs(R).astype(np.float64))
+    bound = np.maximum(bound, k * 2.0 ** -24 * (np.abs(L).astype(np.float64) @ np.abs(R).astype(np.float64)))
+    assert np.all(np.abs(got[0] - ref) <= bound)

@@ -169,11 +169,21 @@ static bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
 // 512- and 256-wide layers, 64 x 128 for the 128-wide one (both with 32-row
 // k-tiles, so that the k-loop's barrier sits between two chunks) and
 // 32 x 128 for the narrow heads (measured on gfx950 at 24,576 rows).
+// Most slices of a reduction of kt k-tiles: a slice is bound by its serial
+// chain of k-tiles (2 us each), so a short reduction is cut down to slices of
+// two k-tiles (updates of 20 steps at 384 / 960 / 2,400 rows a minibatch: 3.61 /
+// 3.45 / 3.55 ms with at least eight, 2.58 / 2.67 / 3.24 with three, 2.46 / 2.61 /
+// 3.24 with two, 2.39 / 2.66 / 3.31 with one), a long one to slices of eight,
+// which bounds the partials that the second pass reads. Reductions of up to 128
+// stay whole: the small-K variants run them in one round of loads.
+constexpr int kUnslicedK = 128;
+inline long long max_slices(long long kt) { return std::max({1LL, kt / 8, std::min(kt / 2, 64LL)}); }
+
 // The three-piece bf16 variant (gemm_split.hip) of a product, or -1 where the
 // fp32 tiles stay. Its 128 x 128 tiles pay once enough of them are in flight;
 // fewer are bound by one block's serial chain (2 us per k-tile), which the
 // smaller fp32 tiles shorten. Launches of an actor + critic pair, us, fp32 vs
-// three-piece: forward 2,000 x 512 x 128 13 / 16, 3,000 x 256 x 512 29 / 34,
+// three-piece: forward 2,000 x 512 x 128 13 / 16, 2,000 x 512 x 64 9 / 13, 3,000 x 256 x 512 29 / 34,
 // 4,500 x 256 x 512 37 / 33, 24,576 x 256 x 512 108 / 79, 24,576 x 512 x 128
 // 70 / 49; a layer's backward 1,000 x 512 x 256 43 / 28 + 26, 2,000 51 / 33,
 // 24,576 222 / 151; input-layer weight gradient 512 x 128 x 24,576 63 / 48.
@@ -183,10 +193,11 @@ static int pick_split(const zl_ctx* c, int M, int N, int K, int lay, int epi, bo
   if (!c || !c->split_gemm || lay == L_AM_BK) return -1;
   const long long tiles = cdiv(M, 128) * cdiv(N, 128);
   if (2LL * M * N < tiles * 128 * 128) return -1;
-  // Split-K slices of at least eight k-tiles count as blocks.
-  const long long slices = epi == zk::kEpiStore ? std::max<long long>(1, std::min<long long>(cdiv(256, tiles), K / 256)) : 1;
+  // Split-K slices count as blocks.
+  const long long slices =
+      epi == zk::kEpiStore ? std::min(cdiv(256, tiles), max_slices(K / 32)) : 1;
   long long least = 48;
-  if (lay == L_AK_BK && epi != zk::kEpiStore) least = M > 2048 ? 64 : LLONG_MAX;
+  if (lay == L_AK_BK && epi != zk::kEpiStore) least = M <= 2048 ? LLONG_MAX : K <= 64 ? 192 : 64;
   if (lay == L_AK_BN && epi != zk::kEpiEluGrad) least = 256;
   if (tiles * slices < least) return -1;
   switch (lay) {
@@ -343,16 +354,15 @@ int gemm_splits(const zl_ctx* c, int M, int N, int K, bool a_kc, bool b_kc, int 
     // Deep-K, few-tile shapes (the weight gradients, K = batch rows) would
     // leave most CUs idle: slice K so the grid reaches the split-K target
     // (256 = one workgroup per CU: more slices buy no speed in the GEMM at
-    // 24,576 rows and cost reduction traffic), keeping at least 8 k-tiles
-    // per slice.
+    // 24,576 rows and cost reduction traffic), within max_slices.
     int target = c ? c->splitk_target : 256;
-    if (tiles >= target || kt < 16) return 1;
+    if (tiles >= target || K <= kUnslicedK) return 1;
     // Tiles narrower than 128 columns (the odd-width input layers, launched
     // alone) whose slices would run past 16 k-tiles aim at two workgroups
     // per CU (the trainer actor's 256 x 288 input layer: 59.0 -> 46.8 us;
     // the critic's 512 x 64, 12 k-tiles per slice, stays: 24.5 us).
     if (g.bn < 128 && cdiv(kt, cdiv(target, tiles)) > 16) target *= 2;
-    s = std::min<long long>(cdiv(target, tiles), std::max<long long>(1, kt / 8));
+    s = std::min(cdiv(target, tiles), max_slices(kt));
   }
   s = std::max<long long>(1, std::min(s, kt));
   const long long per = cdiv(kt, s);
@@ -379,7 +389,7 @@ size_t gemm_ws_floats(const zl_ctx* c, int M, int N, int K, bool a_kc, bool b_kc
         return;
       }
       const long long target = 2LL * (c ? c->splitk_target : 256);
-      s = std::max(s, std::min<long long>(cdiv(target, cdiv(M, g.bm) * cdiv(N, g.bn)), std::max<long long>(1, kt / 8)));
+      s = std::max(s, std::min(cdiv(target, cdiv(M, g.bm) * cdiv(N, g.bn)), max_slices(kt)));
     }
   };
   const int split = pick_split(c, M, N, K, lay, epi, true);
