@@ -21,23 +21,131 @@ namespace zk {
 constexpr int kPolicyPitch = kPolicyMaxWidth + 4;  // LDS row pitch of an activation tile
 constexpr int kPolicyWaves = kPolicyThreads / 64;
 constexpr int kPolicyMaxTiles = kPolicyMaxWidth / 16 / kPolicyWaves;  // 16-column tiles per wave
-constexpr int kPolicyPass = 2;  // 16-wide chunks whose loads are issued together
-static_assert(kPolicyRows == 16 && kPolicyThreads >= 32 * kPolicyRows, "one 16-row MFMA tile; a 32-lane group per row");
+// float4 weight chunks a wavefront keeps in flight: one tile takes them as a
+// ring of four chunks, two tiles as rings of two, within the 64 VGPRs of two
+// blocks per CU. Eight (98 VGPRs, one block per CU) measured no faster: 23.7 vs
+// 22.9 us per step at 64 rows, 45.8 vs 40.7 at 4,096.
+constexpr int kPolicyDepth = 4;
+static_assert(kPolicyRows == 16 && kPolicyWaves == kPolicyRows && kPolicyThreads >= 32 * kPolicyRows,
+              "one 16-row MFMA tile; a wavefront per input row; a 32-lane group per row");
+static_assert(kPolicyMaxTiles <= 2, "one or two tiles per wavefront");
 
+// This lane's float4 of a tile's chunk c: 32-bit byte offsets from the uniform
+// base, one register per address.
+__device__ __forceinline__ float4 policy_chunk(const float* Wp, unsigned w, int c) {
+  return *reinterpret_cast<const float4*>(reinterpret_cast<const char*>(Wp) + (w + 1024u * c));
+}
+
+// A wavefront's nu tiles of one layer, src [16 x 16 kc] in LDS times the packed
+// chunks at w[u] (bytes from Wp). Issue the first chunks of every tile, without
+// a branch (a wavefront with no tile re-reads chunks of another's), so that the
+// loads stay in flight over the code between the layers ...
+__device__ __forceinline__ void policy_prime(float4 (&ring)[kPolicyDepth], const float* Wp, const unsigned (&w)[2], int nu,
+                                             int kc) {
+#pragma unroll
+  for (int i = 0; i < kPolicyDepth; ++i) {
+    const int j = nu == 2 ? i / 2 : i;
+    ring[i] = policy_chunk(Wp, nu == 2 ? w[i & 1] : w[0], min(j, kc - 1));
+  }
+}
+
+// ... then multiply chunk by chunk, each slot refilled D chunks ahead as soon as
+// it is read (past the end: the last chunk again, never used).
+template <int TU>
+__device__ __forceinline__ void policy_sum(floatx4 (&acc)[2], float4 (&ring)[kPolicyDepth], const float* Wp,
+                                           const unsigned (&w)[2], int kc, const float* src) {
+  constexpr int D = kPolicyDepth / TU;
+  auto step = [&](int c, int j) {
+    const float4 a = *reinterpret_cast<const float4*>(src + 16 * c);
+#pragma unroll
+    for (int u = 0; u < TU; ++u) {
+      const float4 b = ring[j * TU + u];
+      acc[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(a.x, b.x, acc[u], 0, 0, 0);
+      acc[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(a.y, b.y, acc[u], 0, 0, 0);
+      acc[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(a.z, b.z, acc[u], 0, 0, 0);
+      acc[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(a.w, b.w, acc[u], 0, 0, 0);
+    }
+  };
+  int c0 = 0;
+  for (; c0 + D < kc; c0 += D) {
+#pragma unroll
+    for (int j = 0; j < D; ++j) {
+      step(c0 + j, j);
+      const int c = min(c0 + j + D, kc - 1);
+#pragma unroll
+      for (int u = 0; u < TU; ++u) ring[j * TU + u] = policy_chunk(Wp, w[u], c);
+      __builtin_amdgcn_sched_barrier(0);  // else all refills move behind the last product
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < D; ++j)
+    if (c0 + j < kc) step(c0 + j, j);
+}
+
+// What bounds it: up to a few hundred rows a block is alone on its CU and its
+// 0.93 MB of weights (headline actor) arrive one dependent round of loads
+// after another; the fp32 MFMAs alone take 12 us, and 24 us at 4,096 rows (two
+// blocks per CU). The loads therefore run as a ring that is refilled slot by
+// slot, a layer's first chunks and its bias are on their way over the epilogue
+// and the barrier of the layer before, and the input rows and log_std travel
+// with the normaliser's statistics. A step of both headline nets: 28.5 -> 22.9 us
+// at 64 rows, 50.2 -> 40.7 us at 4,096.
 __device__ void policy_body(const PolicyArgs& p) {
   __shared__ __align__(16) float act[2][kPolicyRows * kPolicyPitch];
   __shared__ float s_mu[kPolicyMaxWidth], s_sd[kPolicyMaxWidth];
   __shared__ float s_term[kPolicyThreads];
   __shared__ float s_ls[32], s_sdv[32];
   const PolicyNet& q = p.net[blockIdx.y];
-  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const int t = threadIdx.x, lane = t & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
   const int lr = lane & 15, lg = lane >> 4;
   const long long r0 = (long long)blockIdx.x * kPolicyRows;
   const int nr = (int)min((long long)kPolicyRows, p.rows - r0);
   const int od = q.dims[0];
   const int k0w = (od + 15) & ~15;  // layer 0's reduction width (zero past od)
 
-  // Inputs: rows past nr and columns in [od, k0w) are zero.
+  // This wave's 16-column tiles of a layer: slots wave, wave + kPolicyWaves < nt,
+  // slot s on tile (s + rot) % nt, rotated per block so that concurrent
+  // blocks read different weight tiles (measured within 1 % of no rotation).
+  float4 ring[kPolicyDepth];
+  int tile[2];
+  unsigned woff[2];
+  float bias[2];
+  int nu = 0;
+  auto begin_layer = [&](int l) {
+    const int nt = (q.dims[l + 1] + 15) / 16;
+    const int kc = (l == 0 ? k0w : q.dims[l]) / 16;
+    const int rot = (int)(blockIdx.x % (unsigned)nt);
+    nu = wave + kPolicyWaves < nt ? 2 : wave < nt ? 1 : 0;  // uniform over the wavefront
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int s = wave + kPolicyWaves * u + rot;
+      tile[u] = u >= nu ? 0 : s >= nt ? s - nt : s;
+      woff[u] = 4u * (tile[u] * kc * 256 + 4 * lane);
+    }
+    // The biases first: the ring's own order of arrival then stays exact.
+    const float* bl = p.params + q.b_off[l];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) bias[u] = bl[(unsigned)min(16 * tile[u] + lr, q.dims[l + 1] - 1)];
+    const float* Wp = q.wp + q.wp_off[l];
+    policy_prime(ring, Wp, woff, nu, kc);
+  };
+  begin_layer(0);
+  const bool sampling = blockIdx.y == 0 && p.sample;
+
+  // Inputs, a row per wavefront: rows past nr and columns in [od, k0w) are zero.
+  // The row's loads go out before the wait for the normaliser's statistics.
+  constexpr int kIn = kPolicyMaxWidth / 64;
+  float xin[kIn];
+#pragma unroll
+  for (int i = 0; i < kIn; ++i) {
+    const int c = lane + 64 * i;
+    xin[i] = wave < nr && c < od ? q.x[(r0 + wave) * q.ldx + c] : 0.f;
+  }
+  if (sampling && t < p.A) {
+    s_ls[t] = p.log_std[t];
+    s_sdv[t] = expf(s_ls[t]);
+  }
   if (q.norm) {
     const float count = q.norm[2 * od];
     for (int c = t; c < od; c += kPolicyThreads) {
@@ -46,85 +154,42 @@ __device__ void policy_body(const PolicyArgs& p) {
     }
     __syncthreads();
   }
-  for (int e = t; e < kPolicyRows * k0w; e += kPolicyThreads) {
-    const int row = e / k0w, c = e - row * k0w;
-    float v = 0.f;
-    if (row < nr && c < od) {
-      const float x = q.x[(r0 + row) * q.ldx + c];
-      v = q.norm ? clampf((x - s_mu[c]) / s_sd[c], -5.0f, 5.0f) : x;
-    }
-    act[0][row * kPolicyPitch + c] = v;
+#pragma unroll
+  for (int i = 0; i < kIn; ++i) {
+    const int c = lane + 64 * i;
+    if (c >= k0w) break;
+    float v = xin[i];
+    if (q.norm && wave < nr && c < od) v = clampf((v - s_mu[c]) / s_sd[c], -5.0f, 5.0f);
+    act[0][wave * kPolicyPitch + c] = v;
   }
   __syncthreads();
 
   int cur = 0;
   for (int l = 0; l < q.L; ++l) {
-    const int K = l == 0 ? k0w : q.dims[l];
+    const int kc = (l == 0 ? k0w : q.dims[l]) / 16;
     const int N = q.dims[l + 1];
     const bool last = l == q.L - 1;
     const float* Wp = q.wp + q.wp_off[l];
-    const float* bias = p.params + q.b_off[l];
-    const float* src = act[cur];
+    const float* src = act[cur] + lr * kPolicyPitch + 4 * lg;
     float* dst = act[cur ^ 1];
-    const int nt = (N + 15) / 16;
-    // This wave's 16-column tiles: slots wave, wave + kPolicyWaves, ... < nt,
-    // slot s on tile (s + rot) % nt, rotated per block so that concurrent
-    // blocks read different weight tiles (measured within 1 % of no
-    // rotation). The weight loads go out one round per kPolicyPass chunks.
-    const int rot = (int)(blockIdx.x % (unsigned)nt);
-    auto tile_of = [&](int u) {
-      const int s = wave + kPolicyWaves * u + rot;
-      return s >= nt ? s - nt : s;
-    };
-    floatx4 acc[kPolicyMaxTiles];
-    // 32-bit offsets from the uniform Wp: tile T's chunk c is the 256 floats
-    // at (T * kc + c) * 256, this lane's float4 at 4 * lane within them.
-    const int kc = K / 16;
-    int toff[kPolicyMaxTiles];
+    floatx4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+    const int mine = nu, n[2] = {16 * tile[0] + lr, 16 * tile[1] + lr};
+    const float b[2] = {bias[0], bias[1]};
+    if (mine == 2)
+      policy_sum<2>(acc, ring, Wp, woff, kc, src);
+    else if (mine == 1)
+      policy_sum<1>(acc, ring, Wp, woff, kc, src);
+    // The next layer's first weights travel during the epilogue and the barrier.
+    if (!last) begin_layer(l + 1);
 #pragma unroll
-    for (int u = 0; u < kPolicyMaxTiles; ++u) {
-      acc[u] = floatx4{0.f, 0.f, 0.f, 0.f};
-      toff[u] = tile_of(u) * kc * 256 + 4 * lane;
-    }
-    if (wave < nt) {  // uniform over the wavefront
-      for (int kp = 0; kp < K; kp += 16 * kPolicyPass) {
-        float4 av[kPolicyPass], bv[kPolicyPass][kPolicyMaxTiles];
+    for (int u = 0; u < 2; ++u) {
+      if (u >= mine || n[u] >= N) continue;
 #pragma unroll
-        for (int j = 0; j < kPolicyPass; ++j) {
-          const int k = kp + 16 * j + 4 * lg;
-          const bool in = kp + 16 * j < K;  // uniform: K % 16 == 0
-          av[j] = in ? *reinterpret_cast<const float4*>(src + lr * kPolicyPitch + k) : float4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-          for (int u = 0; u < kPolicyMaxTiles; ++u)
-            bv[j][u] = in && wave + kPolicyWaves * u < nt
-                           ? *reinterpret_cast<const float4*>(Wp + (toff[u] + 16 * (kp + 16 * j)))
-                           : float4{0.f, 0.f, 0.f, 0.f};
-        }
-#pragma unroll
-        for (int j = 0; j < kPolicyPass; ++j) {
-          if (kp + 16 * j >= K) break;
-#pragma unroll
-          for (int u = 0; u < kPolicyMaxTiles; ++u) {
-            if (wave + kPolicyWaves * u >= nt) break;
-            acc[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[j].x, bv[j][u].x, acc[u], 0, 0, 0);
-            acc[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[j].y, bv[j][u].y, acc[u], 0, 0, 0);
-            acc[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[j].z, bv[j][u].z, acc[u], 0, 0, 0);
-            acc[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[j].w, bv[j][u].w, acc[u], 0, 0, 0);
-          }
-        }
-      }
-#pragma unroll
-      for (int u = 0; u < kPolicyMaxTiles; ++u) {
-        const int n = 16 * tile_of(u) + lr;
-        if (wave + kPolicyWaves * u >= nt || n >= N) continue;
-        const float b = bias[n];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int row = 4 * lg + r;
-          const float v = last ? acc[u][r] + b : elu(acc[u][r] + b);
-          dst[row * kPolicyPitch + n] = v;
-          if (last && q.out && row < nr) q.out[(r0 + row) * q.ldo + n] = v;
-        }
+      for (int r = 0; r < 4; ++r) {
+        const int row = 4 * lg + r;
+        const float v = last ? acc[u][r] + b[u] : elu(acc[u][r] + b[u]);
+        dst[row * kPolicyPitch + n[u]] = v;
+        if (last && q.out && row < nr) q.out[(r0 + row) * q.ldo + n[u]] = v;
       }
     }
     __syncthreads();
@@ -133,13 +198,8 @@ __device__ void policy_body(const PolicyArgs& p) {
 
   // Sampling (as zk_sample_g32): a 32-lane group per row, lane k on component
   // k; the row's logp terms added in component order by its first lane.
-  if (blockIdx.y != 0 || !p.sample) return;
+  if (!sampling) return;
   const int A = p.A;
-  if (t < A) {
-    s_ls[t] = p.log_std[t];
-    s_sdv[t] = expf(s_ls[t]);
-  }
-  __syncthreads();
   const int g = t / 32, k = t % 32;
   const long long r = r0 + g;
   float term = 0.f;
