@@ -239,3 +239,12 @@ def test_policy_weights_follow_parameter_changes(ctx):
     for h in (other, gac, ref):
         h.close()
     cref.close()
+
+
+@pytest.mark.parametrize("n,ad,cd", [(17, [37, 64, 48, 7], [37, 64, 48, 1]), (300, [1, 16, 32], [45, 512, 1]),
+                                     (8191, [37, 64, 48, 7], [241, 32, 1])])
+def test_fused_policy_step_odd_input_widths(ctx, n, ad, cd):
+    """Input widths whose 16-padded width lies past the weight rows: the
+    packed copy's zeros stand in for the missing columns. Layers of one chunk
+    and of one tile; bit-identical to the layer launches."""
+    test_fused_policy_step_matches_layer_launches(ctx, n, ad, cd)
