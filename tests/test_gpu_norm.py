@@ -190,3 +190,19 @@ def test_bad_arguments_rejected(ctx):
         norm.update(x, 4, ld=7)
     with pytest.raises(ZealotError):
         GpuNormalizer(ctx, 5000)
+
+
+@pytest.mark.parametrize("dim,rows", [(8, 32_768), (9, 32_769), (17, 70_001), (1, 33_000), (4096, 300)])
+def test_update_merge_edges(ctx, dim, rows):
+    """Around one chunk per run of zk_norm_merge (128 runs of 256 rows), columns
+    around a block's eight, one block and hundreds; two updates in a row, so
+    that the second starts from a folded count."""
+    x = obs_rows(rows + dim, rows, dim)
+    norm = GpuNormalizer(ctx, dim)
+    dx = ctx.to_device(x)
+    prior = zo.norm_new(dim)
+    norm.update(dx, rows)
+    check_stats(flat(norm), closed_form(prior, x), dim, f"update {rows} x {dim}")
+    norm.update(dx, rows)
+    assert flat(norm)[2 * dim] == 1 + 2 * rows
+    check_stats(flat(norm), closed_form(prior, np.concatenate([x, x])), dim, f"two updates {rows} x {dim}")

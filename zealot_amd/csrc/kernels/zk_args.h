@@ -436,13 +436,16 @@ struct PolicyArgs {
 // with count 0 is empty (its mean and m2 are zero).
 constexpr int kNormMaxDim = 4096;
 constexpr int kNormChunkRows = 256;    // rows per partial-statistics chunk
-constexpr int kNormFoldThreads = 1024;  // zk_norm_merge / zk_norm_commit block
+constexpr int kNormFoldThreads = 1024;  // zk_norm_commit block
+constexpr int kNormMergeCols = 8;       // zk_norm_merge: columns per block,
+constexpr int kNormMergeRuns = 128;     // threads (runs of chunks) per column; a power of two
 struct NormArgs {
   const float* x;   // [rows x ldx]
   float* out;       // zk_norm_apply: [rows x ldo]
   float* state;     // fold / commit target, zk_norm_apply source, zk_norm_set target
   float* pending;   // zk_norm_commit: folded into state, then emptied
   float* part;      // [nchunks x 2 x dim]: per chunk mean[dim], then M2[dim]
+  int* ticket;      // zk_norm_merge: blocks done, 0 before it (zk_norm_stats clears it)
   long long rows;
   int dim, ldx, ldo, nchunks;
   int rows_per_block;  // zk_norm_apply

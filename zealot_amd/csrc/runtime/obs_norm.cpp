@@ -37,18 +37,20 @@ zl_status zl_norm_update(zl_ctx* c, float* state, int dim, const float* x, int l
   if (rows == 0) return ZL_OK;
   const long long nchunks = cdiv(rows, zk::kNormChunkRows);
   if (nchunks > INT32_MAX / 2) return fail(c, ZL_ERR_INVALID, "zl_norm_update: too many rows");
-  zl_status s = ensure_ws(c, (size_t)nchunks * 2 * dim);
+  zl_status s = ensure_ws(c, (size_t)nchunks * 2 * dim + 1);
   if (s) return s;
   zk::NormArgs a{};
   a.x = x;
   a.state = state;
   a.part = c->ws;
+  a.ticket = reinterpret_cast<int*>(c->ws + (size_t)nchunks * 2 * dim);
   a.rows = rows;
   a.dim = dim;
   a.ldx = ld;
   a.nchunks = (int)nchunks;
   if ((s = launch(c, K_NORM_STATS, (unsigned)nchunks, (unsigned)cdiv(dim, 64), 1, a))) return s;
-  return launch(c, K_NORM_MERGE, 1, 1, 1, a, 0, zk::kNormFoldThreads);
+  return launch(c, K_NORM_MERGE, (unsigned)cdiv(dim, zk::kNormMergeCols), 1, 1, a, 0,
+                zk::kNormMergeCols * zk::kNormMergeRuns);
 }
 
 zl_status zl_norm_commit(zl_ctx* c, float* state, float* pending, int dim) {
