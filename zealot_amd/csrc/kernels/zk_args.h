@@ -341,6 +341,7 @@ struct EluBwdArgs {
   const int* guard;
 };
 
+constexpr int kRowSumWideThreads = 1024;  // zk_row_sum_wide block
 struct RowSumArgs {
   float* out;
   const float* x;

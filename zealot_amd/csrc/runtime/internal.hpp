@@ -28,6 +28,7 @@ enum KernelId : int {
   K_ADV_NORM,
   K_ELU_BACKWARD,
   K_ROW_SUM,
+  K_ROW_SUM_WIDE,
   K_COPY_ROWS,
   K_SAMPLE,
   K_CLAMP,
