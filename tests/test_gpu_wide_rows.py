@@ -1,10 +1,13 @@
-"""Row sums over thousands of columns (zk_row_sum_wide) at the edges of their
-blocks."""
+"""Row sums over thousands of columns (zk_row_sum_wide) and output layers on
+feature-major operands (zk_narrow_f*), at the edges of their blocks; the layers
+of short minibatches (zk_narrow_n1_v, zk_narrow_f22)."""
 
 import numpy as np
 import pytest
 
-from zealot_amd import ops
+from oracle import zl_oracle as zo
+from zealot_amd import ops, synth
+from zealot_amd.rl import GpuMlp
 
 pytestmark = pytest.mark.gpu
 
@@ -25,3 +28,45 @@ def test_row_sum_not_finite(ctx, bad):
     out = ctx.alloc(2)
     ops.row_sum(ctx, out, ctx.to_device(x), 2, 9000)
     assert np.array_equal(out.numpy(), np.array([9000, bad], np.float32), equal_nan=True)
+
+
+@pytest.mark.parametrize("m", [1, 16, 17, 32])
+@pytest.mark.parametrize("n,k", [(1, 33), (15, 48), (17, 100), (300, 123), (4096, 512), (131, 513), (64, 16 * 8 * 5)])
+def test_feature_major_output_layer(ctx, m, n, k):
+    """C[m x n] = W[m x k] X[k x n] + bias, with and without ELU. Bound: k
+    products and additions in any order, the bias, the activation (|slope| <= 1)."""
+    g = np.random.default_rng(m * 1000 + n + k)
+    w, x, b = (g.standard_normal(s).astype(np.float32) for s in ((m, k), (k, n), (m,)))
+    dw, dx, db, out = ctx.to_device(w), ctx.to_device(x), ctx.to_device(b), ctx.alloc((m, n))
+    z = w.astype(np.float64) @ x + b[:, None]
+    bound = 2.0**-24 * (k + 4) * (np.abs(w).astype(np.float64) @ np.abs(x) + np.abs(b)[:, None] + 1)
+    for act in (False, True):
+        ops.gemm_bias_act(ctx, out, dw, dx, m, n, k, db, 1, act)
+        ref = np.where(z > 0, z, np.expm1(np.minimum(z, 0))) if act else z
+        assert np.all(np.abs(out.numpy() - ref) <= bound)
+
+
+@pytest.mark.parametrize("rows", [1, 63, 64, 65, 383, 384, 385])
+@pytest.mark.parametrize("dims", [[48, 80, 64, 16], [30, 512, 100, 33, 5]])
+def test_short_batches(ctx, rows, dims):
+    """Forward strips and data gradients of up to 384 rows and the row after,
+    widths off the 16 and 32 column tiles; against the oracle with the bar of
+    the layer GEMMs (1e-4 of each tensor's largest value)."""
+    g = np.random.default_rng(rows)
+    params = synth.kaiming_uniform_net(g, dims, 0.1)
+    x = g.standard_normal((rows, dims[0])).astype(np.float32)
+    gout = (g.standard_normal((rows, dims[-1])) / rows).astype(np.float32)
+    mlp = GpuMlp(ctx, dims, rows)
+    mlp.write_weights(params)
+    dx, dg = ctx.to_device(x), ctx.to_device(gout)
+    mlp.forward(dx, rows)
+    ref = zo.mlp_forward(dims, params, x)[-1]
+    assert np.abs(mlp.output(rows) - ref).max() <= 1e-4 * np.abs(ref).max()
+    mlp.backward(dg)
+    got, (ref, _) = mlp.read_grads(), zo.mlp_backward(dims, params, x, gout)
+    o = 0
+    for i, j in zip(dims, dims[1:]):
+        for sz in (j * i, j):
+            a, b = got[o:o + sz], ref[o:o + sz]
+            assert np.abs(a - b).max() <= 1e-4 * np.abs(b).max()
+            o += sz

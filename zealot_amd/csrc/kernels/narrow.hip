@@ -14,8 +14,9 @@
 // the 16-wide chunk k0 carries index k0 + 4 s + c: one float4 load per lane
 // feeds four consecutive MFMAs.
 //
-//   zk_narrow_n*  C[M x N] = A[M x K] . B[N x K]^T (+ bias, ELU), N <= 32
-//                 (the forward of an output layer; A rows may be gathered).
+//   zk_narrow_n*  C[M x N] = A[M x K] . B[N x K]^T (+ bias, ELU), 16 or 32
+//                 columns per block (the forward of an output layer, every
+//                 layer of a short minibatch; A rows may be gathered).
 //   zk_narrow_k   C[M x N] = A[M x K] . B[K x N] (x ELU'(Y)), K <= 32
 //                 (the data gradient through an output layer).
 //   zk_narrow_m*  C[M x N] = A^T . B over K rows, A stored [K x M] (M <= 32),
@@ -23,6 +24,9 @@
 //                 blockIdx.x slices the rows (fixed-order partials reduced
 //                 by zk_splitk_reduce, like split-K), blockIdx.y takes 64
 //                 columns; also the row sums of A (the bias gradient).
+//   zk_narrow_f*  C[M x N] = A[M x K] . B[K x N] (+ bias, ELU, x ELU'(Y)), few
+//                 tiles (the feature-major forward of an output layer, the
+//                 data gradients of a short minibatch): wavefronts split K.
 #pragma once
 #include "common.hip"
 
@@ -32,6 +36,7 @@ namespace zk {
 // of the weight-gradient form.
 constexpr int kNarrowWaves = 4;
 constexpr int kNarrowMTiles = 4;
+constexpr int kNarrowFWaves = 8;  // wavefronts over K of the feature-major form
 
 // The epilogue shared with the tiled kernels (gemm_mfma.hip).
 __device__ __forceinline__ float narrow_epilogue(const GemmArgs& p, float v, int m, int n) {
@@ -47,7 +52,7 @@ __device__ __forceinline__ float narrow_epilogue(const GemmArgs& p, float v, int
   return v;
 }
 
-// C = A . B^T, both K-contiguous, N <= 16 * NT. VEC: K % 16 == 0 and both
+// C = A . B^T, both K-contiguous, 16 * NT columns per block. VEC: K % 16 == 0 and both
 // operands' rows 16-byte aligned (float4 loads); otherwise element loads
 // with the K tail zeroed. K is walked in passes of 128: all loads of a pass
 // are issued before its first MFMA, so a strip costs one memory latency per
@@ -60,12 +65,14 @@ __device__ __forceinline__ void narrow_n_body(const GemmArgs& p) {
   const int row0 = (blockIdx.x * kNarrowWaves + (threadIdx.x >> 6)) * 16;
   if (row0 >= p.M) return;  // uniform over the wavefront
   const int lr = lane & 15, lg = lane >> 4;
+  const int n0 = 16 * NT * blockIdx.y;
+  if (n0 >= p.N) return;  // a paired problem's wider grid
   const int m = min(row0 + lr, p.M - 1);
   const long long sr = p.permA ? p.permA[m] : m;
   const float* a = p.A + sr * p.lda;
   const float* b[NT];
 #pragma unroll
-  for (int t = 0; t < NT; ++t) b[t] = p.B + (long long)min(16 * t + lr, p.N - 1) * p.ldb;
+  for (int t = 0; t < NT; ++t) b[t] = p.B + (long long)min(n0 + 16 * t + lr, p.N - 1) * p.ldb;
   floatx4 acc[NT];
 #pragma unroll
   for (int t = 0; t < NT; ++t) acc[t] = floatx4{0.f, 0.f, 0.f, 0.f};
@@ -115,7 +122,7 @@ __device__ __forceinline__ void narrow_n_body(const GemmArgs& p) {
   }
 #pragma unroll
   for (int t = 0; t < NT; ++t) {
-    const int n = 16 * t + lr;
+    const int n = n0 + 16 * t + lr;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int mm = row0 + 4 * lg + r;
@@ -314,6 +321,98 @@ __device__ __forceinline__ void narrow_m_body(const GemmArgs& p) {
   }
 }
 
+// C = A . B with few tiles: a block takes 16 MT rows x 16 NT columns of C, its
+// wavefronts contiguous runs of the K chunks (loads of four chunks issued
+// together), and their partials are added in wavefront order from LDS. On 64 x 64
+// tiles such a product is a handful of blocks, each serial over K: 18.1 us for
+// 29 x 4,096 x 512 (64 blocks), now 6.7 (256 blocks, 8.4 MB of B at 1.3 TB/s:
+// a launch, one trip to memory, the fold).
+// VEC: K % 16 == 0 and A's rows 16-byte aligned.
+template <int MT, int NT, bool VEC>
+__device__ __forceinline__ void narrow_f_body(const GemmArgs& p, float (&red)[kNarrowFWaves][MT * NT][4][64]) {
+  constexpr int P = 4;  // chunks whose loads are issued together
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const int lr = lane & 15, lg = lane >> 4;
+  const int n0 = blockIdx.x * 16 * NT, m0 = blockIdx.y * 16 * MT;
+  if (n0 >= p.N || m0 >= p.M) return;  // uniform: a paired problem's larger grid
+  const float* b[NT];
+#pragma unroll
+  for (int u = 0; u < NT; ++u) b[u] = p.B + min(n0 + 16 * u + lr, p.N - 1);
+  const float* a[MT];
+#pragma unroll
+  for (int i = 0; i < MT; ++i) {
+    const int m = min(m0 + 16 * i + lr, p.M - 1);
+    a[i] = p.A + (long long)(p.permA ? p.permA[m] : m) * p.lda;
+  }
+  floatx4 acc[MT * NT];
+#pragma unroll
+  for (int i = 0; i < MT * NT; ++i) acc[i] = floatx4{0.f, 0.f, 0.f, 0.f};
+  const int K = p.K, kc = (K + 15) / 16, per = (kc + kNarrowFWaves - 1) / kNarrowFWaves;
+  const int c1 = min(kc, (wave + 1) * per);
+  for (int c = wave * per; c < c1; c += P) {
+    float av[P][MT][4], bv[P][NT][4];
+#pragma unroll
+    for (int j = 0; j < P; ++j) {
+      const int k = 16 * (c + j) + 4 * lg;
+      const bool in = c + j < c1;  // uniform over the wavefront
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        const bool ins = in && (VEC || k + s < K);
+        const long long row = (long long)(!ins ? 0 : p.permB ? p.permB[k + s] : k + s) * p.ldb;
+#pragma unroll
+        for (int u = 0; u < NT; ++u) bv[j][u][s] = ins ? b[u][row] : 0.f;
+      }
+#pragma unroll
+      for (int i = 0; i < MT; ++i) {
+        if constexpr (VEC) {
+          const float4 v = in ? *reinterpret_cast<const float4*>(a[i] + k) : float4{0.f, 0.f, 0.f, 0.f};
+          av[j][i][0] = v.x;
+          av[j][i][1] = v.y;
+          av[j][i][2] = v.z;
+          av[j][i][3] = v.w;
+        } else {
+#pragma unroll
+          for (int s = 0; s < 4; ++s) av[j][i][s] = in && k + s < K ? a[i][k + s] : 0.f;
+        }
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < P; ++j)
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+#pragma unroll
+          for (int u = 0; u < NT; ++u)
+            acc[i * NT + u] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[j][i][s], bv[j][u][s], acc[i * NT + u], 0, 0, 0);
+  }
+#pragma unroll
+  for (int i = 0; i < MT * NT; ++i)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) red[wave][i][r][lane] = acc[i][r];
+  __syncthreads();
+  for (int e = t; e < MT * NT * 256; e += 64 * kNarrowFWaves) {
+    const int i = e >> 8, r = (e >> 6) & 3, l = e & 63;
+    const int m = m0 + 16 * (i / NT) + 4 * (l >> 4) + r, n = n0 + 16 * (i % NT) + (l & 15);
+    float v = 0.f;
+#pragma unroll
+    for (int w = 0; w < kNarrowFWaves; ++w) v += red[w][i][r][l];
+    if (m < p.M && n < p.N) p.C[(long long)m * p.ldc + n] = narrow_epilogue(p, v, m, n);
+  }
+}
+
+template <int MT, int NT>
+__device__ __forceinline__ void narrow_f(const GemmBatch& b) {
+  __shared__ float red[kNarrowFWaves][MT * NT][4][64];
+  if ((int)blockIdx.z >= b.count) return;
+  const GemmArgs& p = b.g[blockIdx.z];
+  if (p.guard && *p.guard == 0) return;
+  if (p.vecA && p.K % 16 == 0)
+    narrow_f_body<MT, NT, true>(p, red);
+  else
+    narrow_f_body<MT, NT, false>(p, red);
+}
+
 }  // namespace zk
 
 // grid.z = problem of the batch (one slice per problem: zper = 1).
@@ -330,3 +429,7 @@ ZK_NARROW(zk_narrow_n2_s, (zk::narrow_n_body<2, false>))
 ZK_NARROW(zk_narrow_k, zk::narrow_k_body)
 ZK_NARROW(zk_narrow_m1, zk::narrow_m_body<1>)
 ZK_NARROW(zk_narrow_m2, zk::narrow_m_body<2>)
+
+extern "C" __global__ __launch_bounds__(64 * zk::kNarrowFWaves) void zk_narrow_f1(zk::GemmBatch b) { zk::narrow_f<1, 1>(b); }
+extern "C" __global__ __launch_bounds__(64 * zk::kNarrowFWaves) void zk_narrow_f2(zk::GemmBatch b) { zk::narrow_f<2, 1>(b); }
+extern "C" __global__ __launch_bounds__(64 * zk::kNarrowFWaves) void zk_narrow_f22(zk::GemmBatch b) { zk::narrow_f<2, 2>(b); }

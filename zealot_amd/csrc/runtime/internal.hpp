@@ -62,8 +62,9 @@ enum KernelId : int {
 // Kernel family of a GEMM variant: LDS-tiled (gemm_mfma.hip), three-piece bf16
 // (gemm_split.hip, launched and split over K like the tiled ones) or one of the
 // register-resident narrow kernels (narrow.hip): N <= 32 (forward of an
-// output layer), K <= 32 (its data gradient), M <= 32 (its weight gradient).
-enum GemmKind : int { G_TILED = 0, G_NARROW_N = 1, G_NARROW_K = 2, G_NARROW_M = 3, G_SPLIT = 4 };
+// output layer), K <= 32 (its data gradient), M <= 32 (its weight gradient, and
+// its forward on feature-major operands).
+enum GemmKind : int { G_TILED = 0, G_NARROW_N = 1, G_NARROW_K = 2, G_NARROW_M = 3, G_SPLIT = 4, G_NARROW_F = 5 };
 inline bool is_tiled(int kind) { return kind == G_TILED || kind == G_SPLIT; }
 
 // One GEMM variant: operand orientation, tile (for the narrow kernels: rows
@@ -84,6 +85,8 @@ struct GemmKernel {
 constexpr int kNarrowRows = 64;
 constexpr int kNarrowKCols = 32;
 constexpr int kNarrowCols = 64;
+constexpr int kShortRows = 384;   // rows up to which a minibatch's layers are latency-bound
+constexpr int kNarrowFCols = 16;  // columns per block of the feature-major forward
 constexpr int kNarrowSliceQuantum = 64;
 
 extern const char* const kFixedNames[K_GEMM_BASE];

@@ -76,6 +76,9 @@ const GemmKernel kGemmTable[] = {
     {"zk_narrow_k", true, false, kNarrowRows, kNarrowKCols, 32, 256, false, G_NARROW_K},
     {"zk_narrow_m1", false, false, 16, kNarrowCols, 16, 256, false, G_NARROW_M},
     {"zk_narrow_m2", false, false, 32, kNarrowCols, 16, 256, false, G_NARROW_M},
+    {"zk_narrow_f1", true, false, 16, kNarrowFCols, 16, 512, false, G_NARROW_F},
+    {"zk_narrow_f2", true, false, 32, kNarrowFCols, 16, 512, false, G_NARROW_F},
+    {"zk_narrow_f22", true, false, 32, 32, 16, 512, false, G_NARROW_F},
 };
 const int kGemmCount = (int)(sizeof(kGemmTable) / sizeof(kGemmTable[0]));
 
@@ -235,6 +238,32 @@ static int pick_fp32(const zl_ctx* c, int M, int N, int K, bool a_kc, bool b_kc,
                      bool vec_b) {
   const int lay = layout_of(a_kc, b_kc);
   const bool forced = c && c->force_gemm[lay] >= 0;
+  if (!forced && (!c || c->narrow) && lay == L_AK_BN && K > 32 && epi != zk::kEpiStore) {
+    const long long tiles = cdiv(M, 32) * cdiv(N, 32);
+    if (epi == zk::kEpiEluGrad) {
+      // Data gradients of a short minibatch: per minibatch of the headline nets
+      // 4-7 us less than the 64 x 64 tiles at 64-384 rows, 7 us more at 768.
+      if (M <= kShortRows && tiles <= 192) return gemm_id("zk_narrow_f22");
+    } else {
+      // Feature-major layers with few tiles, against the 64 x 64 ones: 29 x
+      // 4,096 x 512 18.1 -> 6.7 us, 512 x 512 x 512 17.3 -> 9.1 us, 128 x
+      // 4,096 x 512 (512 tiles) 17.4 -> 13.6 us; past two tiles per CU, or
+      // one where K <= 128, slower (256 x 4,096: 24.2 vs 18.1 us at K =
+      // 512, 512 x 1,024 x 123: 10.8 vs 8.6). Up to 16 rows 16-column
+      // blocks win at any length (12 x 24,576: 6.7-23.6 vs 7.3-25.7 us for K =
+      // 64-512), up to 32 rows while they give a CU one (29 x 4,096 x 512:
+      // 6.7 vs 8.5 us on 32-column blocks, 29 x 8,192: 11.8 vs 8.6).
+      if (M <= 16) return gemm_id("zk_narrow_f1");
+      if (M <= 32 && N <= 4096) return gemm_id("zk_narrow_f2");
+      if (tiles <= (K > 128 ? 512 : 256)) return gemm_id("zk_narrow_f22");
+    }
+  }
+  // Forwards of a short minibatch: a 16 x 16 strip per wavefront instead of
+  // the serial k-tiles of 32 x 64 tiles (per minibatch of the headline nets
+  // 5 us less at 384 rows, 3 us more at 768).
+  if (!forced && (!c || c->narrow) && lay == L_AK_BK && vec && K % 16 == 0 && N > 32 && epi != zk::kEpiStore &&
+      M <= kShortRows && cdiv(M, kNarrowRows) * cdiv(N, 16) <= 192)
+    return gemm_id("zk_narrow_n1_v");
   // K <= 128 with B float4-aligned: one round of loads for the whole K
   // extent (the single 4096 x 123 -> 512 feature-major layer, whose weight
   // rows of 123 floats are not float4-aligned).
@@ -442,7 +471,10 @@ static zl_status plan_gemm(zl_ctx* c, const GemmDesc& d, GemmPlan& P) {
     P.splits = 1;
     P.per = 0;
     P.gx = (unsigned)cdiv(d.M, kNarrowRows);
-    P.gy = g.kind == G_NARROW_K ? (unsigned)cdiv(d.N, kNarrowKCols) : 1u;
+    P.gy = (unsigned)cdiv(d.N, g.bn);
+  } else if (g.kind == G_NARROW_F) {
+    P.gx = (unsigned)cdiv(d.N, g.bn);
+    P.gy = (unsigned)cdiv(d.M, g.bm);
   } else if (g.kind == G_NARROW_M) {
     P.per = narrow_rows_per_slice(c, d.N, d.K, d.epi);
     P.splits = (int)cdiv(std::max(d.K, 1), P.per);
@@ -502,13 +534,15 @@ static zl_status plan_batch(zl_ctx* c, const GemmDesc* d, int n, BatchLaunch& L,
     zl_status s = plan_gemm(c, *live[i], P[i]);
     if (s) return s;
   }
-  // Narrow kernels size one grid for both problems, so only problems of one
-  // shape share such a launch. (Tiled kernels give each problem its own
-  // block range, so the actor's and the critic's layer share a launch
-  // whatever their shapes.)
-  const bool narrow_pair = nl == 2 && !is_tiled(kGemmTable[P[0].kid - K_GEMM_BASE].kind) &&
-                           !is_tiled(kGemmTable[P[1].kid - K_GEMM_BASE].kind);
-  if (narrow_pair &&
+  // Narrow kernels size one grid for both problems. Those that return on
+  // blocks past a problem's rows and columns (zk_narrow_n*, zk_narrow_f*) take
+  // problems of different shapes; the others only problems of one. (Tiled
+  // kernels give each problem its own block range, so the actor's and the
+  // critic's layer share a launch whatever their shapes.)
+  auto kind = [&](int i) { return kGemmTable[P[i].kid - K_GEMM_BASE].kind; };
+  const bool narrow_pair = nl == 2 && !is_tiled(kind(0)) && !is_tiled(kind(1));
+  const bool bounded = narrow_pair && kind(0) == kind(1) && (kind(0) == G_NARROW_N || kind(0) == G_NARROW_F);
+  if (narrow_pair && !bounded &&
       (live[0]->M != live[1]->M || live[0]->N != live[1]->N || live[0]->K != live[1]->K))
     return ZL_OK;
   // A pair whose members differ only in exact fit runs as one launch of
