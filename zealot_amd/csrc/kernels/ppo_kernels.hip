@@ -661,7 +661,7 @@ __device__ void row_sum_body(const RowSumArgs& p) {
   float s = 0.f;
   for (int c = threadIdx.x; c < p.cols; c += kThreads) s += p.x[(long long)r * p.ldx + c];
   const float tot = block_sum(s, red);
-  if (threadIdx.x == 0) p.out[r] = tot;
+  if (threadIdx.x == 0) (p.out2 && r >= p.split ? p.out2[r - p.split] : p.out[r]) = tot;
 }
 
 // Rows of thousands of values: kRowSumWideThreads per row, eight loads in flight

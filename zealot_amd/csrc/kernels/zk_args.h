@@ -347,6 +347,8 @@ struct RowSumArgs {
   const float* x;
   int rows, cols, ldx;
   const int* guard;
+  float* out2;  // rows from `split` on go to out2[row - split] (nullable: all to out)
+  int split;
 };
 
 struct CopyRowsArgs {

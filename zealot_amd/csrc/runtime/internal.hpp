@@ -291,8 +291,10 @@ zl_status launch_reduce_all(zl_ctx* c, const zk::ReduceSeg* segs, int nseg, floa
 // lanes and grid from the shape. `r.lanes` is set here.
 zl_status launch_splitk_reduce(zl_ctx* c, zk::SplitReduceArgs& r);
 zl_status ensure_ws(zl_ctx* c, size_t floats);
-// out[k] = sum over b of part[k * blocks + b], k < width (zk_row_sum).
-zl_status reduce_rows(zl_ctx* c, const float* part, int width, int blocks, float* out);
+// out[k] = sum over b of part[k * blocks + b], k < width (zk_row_sum); with out2,
+// components from `split` on go to out2[k - split].
+zl_status reduce_rows(zl_ctx* c, const float* part, int width, int blocks, float* out,
+                      float* out2 = nullptr, int split = 0);
 // Sampling + logp (zk_sample_g32 / _g64 for A <= 32 / 64, else zk_sample).
 zl_status launch_sample(zl_ctx* c, const zk::SampleArgs& a);
 
