@@ -221,6 +221,41 @@ def test_head_tile_schedules_match_unfused(ctx, n, shuffled):
         assert abs(fs[key] - us[key]) <= 1e-5 * max(1.0, abs(us[key])), key
 
 
+@pytest.mark.parametrize("n", [600, 3001])
+def test_logp_old_not_finite(ctx, n):
+    """An infinite old log-probability makes a sample's ratio 0 (+inf) or
+    infinite (-inf: clipped where adv > 0): the sample drops out of the
+    gradients and its surrogate is 0, or the clip bound times adv. zk_head and
+    the separate loss kernels (ZL_FUSED_HEAD=0) against the oracle, with the
+    bar of the other gradients."""
+    ad, cd = [40, 256, 128, 12], [40, 256, 128, 1]
+    g = np.random.default_rng(41)
+    actor = synth.kaiming_uniform_net(g, ad, 0.1)
+    critic = synth.kaiming_uniform_net(g, cd, 0.1)
+    batch, log_std = make_batch(n, ad, cd, actor, critic, seed=6)
+    move_off_branch_boundaries(batch, ad, cd, actor, critic, log_std)
+    for row, lp, adv in ((5, np.inf, 0.7), (70, -np.inf, 1.3), (n - 1, np.inf, -0.4)):
+        batch["logp_old"][row], batch["adv"][row] = lp, adv
+    db = DeviceBatch(ctx, batch["obs"], batch["obs"], batch["action"], batch["mean_old"],
+                     batch["logp_old"], batch["value_old"], batch["adv"], batch["ret"])
+    ra, rc, rl, rs = zo.minibatch_grads(ad, cd, actor, critic, log_std, batch, np.arange(n), 0.2, 0.01, 1.0)
+    assert np.isfinite(ra).all() and np.isfinite(rs).all()
+    for fused in (True, False):
+        if not fused:
+            os.environ["ZL_FUSED_HEAD"] = "0"
+        try:
+            gac = GpuActorCritic(ctx, ad, cd, n)
+        finally:
+            os.environ.pop("ZL_FUSED_HEAD", None)
+        gac.set_params(actor, critic, log_std, 1e-3)
+        ga, gc, gl, st = gac.minibatch_grads(db, PpoConfig(entropy_coef=0.01), 0, n)
+        gac.close()
+        assert all(np.isfinite(x).all() for x in (ga, gc, gl))
+        assert max(per_tensor_err(ad, ga, ra), per_tensor_err(cd, gc, rc), rel_amax(gl, rl)) <= TOL
+        for key, r in zip(("surrogate", "value_loss", "kl"), rs):
+            assert abs(st[key] - r) <= 1e-5 * max(1.0, abs(r)), (fused, key)
+
+
 @pytest.mark.parametrize("n,shuffled", [(3001, True), (24576, False), (24576, True)])
 def test_head_forward_fused_matches_separate(ctx, n, shuffled):
     """zk_head_fwd (the last hidden layer's forward computed tile by tile

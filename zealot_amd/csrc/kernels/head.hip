@@ -103,12 +103,30 @@ __device__ __forceinline__ void head_forward_tile(const HeadNet& q, long long ro
       smem, a, 0, (int)(r0 / kHeadRows), 0, sx);
 }
 
-// Sum over the 32 lanes of a group by a fixed butterfly: every lane ends with
-// the same bits (each step adds two partners).
-__device__ __forceinline__ float group_sum(float v) {
+// Sum over a row's 32 components in component order, every lane of the
+// 32-lane group getting the result: lane k stores its term in the row's LDS
+// slot k (components >= A hold 0, and adding 0 changes no sum), the group's
+// first lane reads the row back as 8 float4 loads and adds them in order, and
+// the two groups' sums (lanes 0 and 32 of the wavefront) are broadcast with
+// v_readlane. LDS instructions of one wavefront execute in order, so no
+// barrier is needed; one reading lane per group instead of 32 keeps the LDS
+// traffic of the losses at 1/32.
+__device__ __forceinline__ float row_sum_ordered(float* srow, int k, float term) {
+  srow[k] = term;
+  float s = 0.f;
+  if (k == 0) {
 #pragma unroll
-  for (int m = 16; m > 0; m >>= 1) v = v + __shfl_xor(v, m, 32);
-  return v;
+    for (int c = 0; c < kHeadMaxActions / 4; ++c) {
+      const float4 v = *reinterpret_cast<const float4*>(srow + 4 * c);
+      s += v.x;
+      s += v.y;
+      s += v.z;
+      s += v.w;
+    }
+  }
+  const float s0 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, s), 0));
+  const float s1 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, s), 32));
+  return (threadIdx.x & 32) ? s1 : s0;
 }
 
 // FWD: 0 reads the tile of the last hidden activations; 1 (masked) / 2
@@ -163,7 +181,6 @@ __device__ void head_actor(const HeadArgs& p, float* smem) {
   };
   if constexpr (FWD == 0) loss_consts();
   const float lo = 1.0f - p.clip, hi = 1.0f + p.clip;
-  const float inv_A = 1.0f / (float)A;
   float gacc = 0.f, sacc = 0.f, kacc = 0.f;
   float klacc = 0.f;  // sum of (mean - mean_old)^2 of component k over the group's rows
   float dbias = 0.f;  // thread t < 32: bias gradient of component t
@@ -252,16 +269,14 @@ __device__ void head_actor(const HeadArgs& p, float* smem) {
     lds_barrier();
 
     // Head forward: rows of tile rt, components 16 * half ...; the k range
-    // in four interleaved chains (16-wide chunks c, c + 4) added pairwise at the end.
+    // in two interleaved chains (even and odd 16-wide chunks) added at the end.
     {
-      floatx4 ch[4];
-#pragma unroll
-      for (int c = 0; c < 4; ++c) ch[c] = floatx4{0.f, 0.f, 0.f, 0.f};
+      floatx4 acc2[2] = {floatx4{0.f, 0.f, 0.f, 0.f}, floatx4{0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
       for (int c16 = 0; c16 < kHeadMaxHidden / 16; ++c16) {
         const float4 af = *reinterpret_cast<const float4*>(sx + (16 * rt + lr) * kHeadPitch + 16 * c16 + 4 * lg);
         const float4 bf = *reinterpret_cast<const float4*>(sw + (16 * half + lr) * kHeadPitch + 16 * c16 + 4 * lg);
-        floatx4& acc = ch[c16 & 3];
+        floatx4& acc = acc2[c16 & 1];
         acc = __builtin_amdgcn_mfma_f32_16x16x4f32(af.x, bf.x, acc, 0, 0, 0);
         acc = __builtin_amdgcn_mfma_f32_16x16x4f32(af.y, bf.y, acc, 0, 0, 0);
         acc = __builtin_amdgcn_mfma_f32_16x16x4f32(af.z, bf.z, acc, 0, 0, 0);
@@ -271,7 +286,7 @@ __device__ void head_actor(const HeadArgs& p, float* smem) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int row = 16 * rt + 4 * lg + r;
-        const float mu = m < A ? ((ch[0][r] + ch[1][r]) + (ch[2][r] + ch[3][r])) + bias_f : 0.f;
+        const float mu = m < A ? (acc2[0][r] + acc2[1][r]) + bias_f : 0.f;
         sd[row * kHeadDPitch + m] = mu;
         if (m < A && row < nr) q.out[(r0 + row) * q.ldo + m] = mu;
       }
@@ -291,13 +306,8 @@ __device__ void head_actor(const HeadArgs& p, float* smem) {
         const float mu = srow[k];
         const float act = in[j].act;
         const float dz = (act - mu) / sdv;
-        // log ratio = sum_k (logp term k - q) - (logp_old - A q) with q =
-        // logp_old / A: the log-probabilities reach a few hundred, where a
-        // running fp32 sum of them leaves 2e-5 of the ratio open; the terms
-        // minus q stay small and logp_old - A q is exact.
-        const float q = in[j].lpo * inv_A;
-        const float lr = group_sum(on ? (-0.5f * dz * dz - ls - kLogSqrt2Pi) - q : 0.f);
-        const float ratio = expf(lr - fmaf(-(float)A, q, in[j].lpo));
+        const float lp = row_sum_ordered(srow, k, on ? -0.5f * dz * dz - ls - kLogSqrt2Pi : 0.f);
+        const float ratio = expf(lp - in[j].lpo);
         const float a = in[j].adv;
         const float surr = fminf(ratio * a, clampf(ratio, lo, hi) * a);
         const bool clipped = (a >= 0.0f && ratio > hi) || (a < 0.0f && ratio < lo);
@@ -313,8 +323,13 @@ __device__ void head_actor(const HeadArgs& p, float* smem) {
         sacc += surr * p.scale;
         if (p.mean_old) {
           const float y = (mu - in[j].mo) * inv_sd;
-          // The mean-only KL (ActorCritic::kl, ppo.rs:327-334).
-          kacc += group_sum(on ? 0.5f * (y * y) : 0.f) * p.scale;
+          // The mean-only KL (ActorCritic::kl, ppo.rs:327-334) is a statistic:
+          // a fixed butterfly over the group is enough (every lane ends with
+          // the same bits: each step adds two equal-valued partners).
+          float kt = on ? 0.5f * (y * y) : 0.f;
+#pragma unroll
+          for (int m = 16; m > 0; m >>= 1) kt = kt + __shfl_xor(kt, m, 32);
+          kacc += kt * p.scale;
           if (p.kl_part && on) {
             const float dmu = mu - in[j].mo;
             klacc += dmu * dmu;
