@@ -146,6 +146,35 @@ def test_split_gemm_network(ctx, rows):
     mlp.close()
 
 
+@pytest.mark.parametrize("n", [384, 3001, 24576])
+def test_minibatch_forward_stays_fp32(ctx, fp32_ctx, n):
+    """The surrogate of a minibatch is a mean of signed terms that nearly
+    cancel: its forward stays on the fp32 kernels, so every statistic and the
+    log_std gradient have the bits of a context without three-piece GEMMs; the
+    weight gradients, which may take them, agree to rounding."""
+    from zealot_amd.rl import DeviceBatch, GpuActorCritic, PpoConfig
+
+    ad, cd = [123, 512, 256, 128, 29], [123, 512, 256, 128, 1]
+    g = np.random.default_rng(n)
+    actor, critic = synth.kaiming_uniform_net(g, ad, 0.1), synth.kaiming_uniform_net(g, cd, 0.1)
+    obs = synth.obs(g, n, 123)
+    args = [obs, obs, synth.normal(g, (n, 29)), synth.normal(g, (n, 29)), synth.normal(g, n) - 60, synth.normal(g, n),
+            synth.normal(g, n), synth.normal(g, n)]
+    out = []
+    for c in (ctx, fp32_ctx):
+        gac = GpuActorCritic(c, ad, cd, n)
+        gac.set_params(actor, critic, np.full(29, -0.5, np.float32), 1e-4)
+        db = DeviceBatch(c, *args)
+        names = used(c, lambda: out.append(gac.minibatch_grads(db, PpoConfig(), 0, n)))
+        assert not any(x.startswith("zk_split_ak_bk") for x in names), names
+        assert any(x.startswith("zk_split_") for x in names) == (c is ctx), names
+        gac.close()
+    (ga, gc, gl, st), (ra, rc, rl, rst) = out
+    assert st == rst and np.array_equal(gl, rl)
+    for a, b in ((ga, ra), (gc, rc)):
+        assert np.linalg.norm(a - b) <= 2e-6 * np.linalg.norm(b)
+
+
 def test_split_gemm_gathered_rows(ctx):
     """A shuffled minibatch of a ragged number of rows (the observation gather
     inside the first layer's forward and weight gradient): the same rows in

@@ -251,6 +251,7 @@ struct GemmDesc {
   int ldy = 0;
   float* rowsum_out = nullptr;  // row sums of A (bias gradient of a wgrad)
   int splits = 0;               // 0: heuristic; only kEpiStore may split
+  bool fp32 = false;            // the fp32 MFMA kernels, also where three-piece ones would be faster
   const int* guard = nullptr;
   float* ws = nullptr;          // split-K scratch (floats); nullptr: context scratch
   size_t ws_floats = 0;
@@ -265,11 +266,9 @@ struct GemmDesc {
 // kvec: every K-contiguous operand can be read as float4 rows (the three-piece
 // variants read the others by elements).
 int pick_gemm(const zl_ctx* c, int M, int N, int K, bool a_kc, bool b_kc, bool vec = true,
-              int epi = zk::kEpiStore, bool vec_b = false, bool kvec = true);
+              int epi = zk::kEpiStore, bool vec_b = false, bool kvec = true, bool fp32_only = false);
 int gemm_splits(const zl_ctx* c, int M, int N, int K, bool a_kc, bool b_kc, int epi,
                 bool vec = true);
-// Whether a row-major forward layer takes the three-piece bf16 kernels.
-bool split_forward(const zl_ctx* c, int M, int N, int K);
 size_t gemm_ws_floats(const zl_ctx* c, int M, int N, int K, bool a_kc, bool b_kc, int epi);
 zl_status run_gemm(zl_ctx* c, const GemmDesc& d);
 // One launch for n (1 or 2) problems that pick the same variant (else n

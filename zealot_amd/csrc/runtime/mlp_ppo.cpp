@@ -206,9 +206,10 @@ static GemmDesc dgrad_desc(const NetLayout& nl, const NetBuffers& nb, const floa
 
 static zl_status net_forward(zl_ctx* c, const NetLayout& nl, const NetBuffers& nb,
                              const float* params, const float* x, int ldx, const int* permx,
-                             int rows, const int* guard, int kx = 0) {
+                             int rows, const int* guard, int kx = 0, bool fp32 = false) {
   for (int l = 0; l < nl.L; ++l) {
-    const GemmDesc d = fwd_desc(nl, nb, params, x, ldx, permx, rows, guard, l, kx);
+    GemmDesc d = fwd_desc(nl, nb, params, x, ldx, permx, rows, guard, l, kx);
+    d.fp32 = fp32;
     zl_status s = run_gemm(c, d);
     if (s) return s;
   }
@@ -247,31 +248,25 @@ struct NetView {
 };
 
 // Forward of both nets, layer by layer, each layer's two GEMMs in one launch
-// when the nets have the same depth (otherwise one after the other).
+// when the nets have the same depth (otherwise one after the other; layers
+// >= 0: only the first ones of equally deep nets). fp32: no three-piece GEMMs.
 static zl_status pair_forward(zl_ctx* c, const NetView v[2], const float* params,
-                              const int* permx, int rows, const int* guard, int layers = -1) {
-  if (layers >= 0 && v[0].nl->L == v[1].nl->L) {
-    for (int l = 0; l < layers; ++l) {
-      GemmDesc d[2];
-      for (int i = 0; i < 2; ++i)
-        d[i] = fwd_desc(*v[i].nl, *v[i].nb, params, v[i].x, v[i].ldx, permx, rows, guard, l, v[i].kx);
-      zl_status s = run_gemm_batch(c, d, 2);
-      if (s) return s;
-    }
-    return ZL_OK;
-  }
+                              const int* permx, int rows, const int* guard, int layers = -1,
+                              bool fp32 = false) {
   if (v[0].nl->L != v[1].nl->L) {
     for (int i = 0; i < 2; ++i) {
       zl_status s = net_forward(c, *v[i].nl, *v[i].nb, params, v[i].x, v[i].ldx, permx, rows, guard,
-                                v[i].kx);
+                                v[i].kx, fp32);
       if (s) return s;
     }
     return ZL_OK;
   }
-  for (int l = 0; l < v[0].nl->L; ++l) {
+  for (int l = 0; l < (layers >= 0 ? layers : v[0].nl->L); ++l) {
     GemmDesc d[2];
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < 2; ++i) {
       d[i] = fwd_desc(*v[i].nl, *v[i].nb, params, v[i].x, v[i].ldx, permx, rows, guard, l, v[i].kx);
+      d[i].fp32 = fp32;
+    }
     zl_status s = run_gemm_batch(c, d, 2);
     if (s) return s;
   }
@@ -902,11 +897,16 @@ zl_status minibatch_pass(zl_ppo* p, const NetView v[2], const int* px, const int
     hfwd = ((uintptr_t)nb.act[l] & 15) == 0 && ((uintptr_t)w2 & 15) == 0 && nb.ld[l] % 4 == 0 &&
            nl.ldw[l] % 4 == 0;
     hfwd_exact = hfwd_exact && nl.dims[l + 1] == zk::kHeadMaxHidden && nl.dims[l] % 32 == 0;
-    // A layer that the three-piece kernels take is faster as its own launch.
-    hfwd = hfwd && !split_forward(c, rows, nl.dims[l + 1], nl.dims[l]);
   }
+  // A minibatch's forward stays on the fp32 MFMAs. Its surrogate is a mean of
+  // signed terms that nearly cancel (of 24,576 of order 1, often below 1e-3), so
+  // another rounding of the policy means moves it by up to 5e-4 of its value
+  // (three-piece forwards, 12 batches of 24,576 rows); in the fp32 kernels' one
+  // order of summation it keeps its bits. The price: 456 -> 500 us per minibatch
+  // of the headline nets (616 with the backward on fp32 MFMAs too). The critic
+  // alone on three-piece products, in launches of its own, was slower: 515.
   zl_status s = pair_forward(c, v, p->params, px, rows, guard,
-                             p->fused_head ? (hfwd ? La - 2 : La - 1) : -1);
+                             p->fused_head ? (hfwd ? La - 2 : La - 1) : -1, true);
   if (s) return s;
   int head_blocks = 0, critic_blocks = 0;
   if (p->fused_head) {

@@ -215,18 +215,14 @@ static int pick_split(const zl_ctx* c, int M, int N, int K, int lay, int epi, bo
   }
 }
 
-bool split_forward(const zl_ctx* c, int M, int N, int K) {
-  return c->force_gemm[L_AK_BK] < 0 && pick_split(c, M, N, K, L_AK_BK, zk::kEpiBiasN, true) >= 0;
-}
-
 static int pick_fp32(const zl_ctx* c, int M, int N, int K, bool a_kc, bool b_kc, bool vec, int epi,
                      bool vec_b);
 
 int pick_gemm(const zl_ctx* c, int M, int N, int K, bool a_kc, bool b_kc, bool vec, int epi,
-              bool vec_b, bool kvec) {
+              bool vec_b, bool kvec, bool fp32_only) {
   const int fp32 = pick_fp32(c, M, N, K, a_kc, b_kc, vec, epi, vec_b);
   const int lay = layout_of(a_kc, b_kc);
-  if ((c && c->force_gemm[lay] >= 0) || fp32 < 0) return fp32;
+  if (fp32_only || (c && c->force_gemm[lay] >= 0) || fp32 < 0) return fp32;
   // Narrow and small-K shapes keep their own kernels.
   const GemmKernel& g = kGemmTable[fp32 - K_GEMM_BASE];
   if (g.kind != G_TILED || strstr(g.name, "xk128")) return fp32;
@@ -456,7 +452,7 @@ static zl_status plan_gemm(zl_ctx* c, const GemmDesc& d, GemmPlan& P) {
   P.vec = va && vb;
   const bool plain = !d.rowsum_out && !d.permA && !d.permB && d.splits <= 1;
   const bool kvec = (!d.a_kc || va) && (!d.b_kc || vb);
-  P.kid = pick_gemm(c, d.M, d.N, d.K, d.a_kc, d.b_kc, P.vec, d.epi, vb && plain, kvec);
+  P.kid = pick_gemm(c, d.M, d.N, d.K, d.a_kc, d.b_kc, P.vec, d.epi, vb && plain, kvec, d.fp32);
   if (P.kid < 0) return fail(c, ZL_ERR_INVALID, "no GEMM variant for this layout");
   const GemmKernel& g = kGemmTable[P.kid - K_GEMM_BASE];
   const bool vec_ok = g.kind == G_SPLIT ? kvec : P.vec;
