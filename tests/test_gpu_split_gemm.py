@@ -107,6 +107,40 @@ def test_split_gemm_special_values(ctx, fp32_ctx, what, lt, rt):
     assert np.all(d <= np.maximum(bound[ok], 0.0) + 1e-45)
 
 
+@pytest.mark.parametrize("what", ["tiny x huge", "subnormal x huge", "tiny row", "tiny column", "subnormal row"])
+@pytest.mark.parametrize("lt,rt", [(False, True), (False, False), (True, False)])
+def test_split_gemm_small_operands(ctx, what, lt, rt):
+    """Operands whose low pieces lie below the bf16 range, alone or beside
+    ordinary rows and columns, with results of ordinary size or not: every row
+    and column as close to float64 as those of ordinary operands. Bound: 6 x
+    19 random-sign roundings of 2^-24 of the running sum are 4e-7 of the root
+    mean square of a row; two pieces alone leave 1e-5."""
+    m, n, k = 1100, 4200, 300
+    g = np.random.default_rng(7)
+    L, R = synth.normal(g, (m, k)), synth.normal(g, (k, n))
+    if what == "tiny x huge":
+        L, R = L * np.float32(2.0**-119), R * np.float32(2.0**60)
+    elif what == "subnormal x huge":
+        L, R = L * np.float32(2.0**-132), R * np.float32(2.0**80)
+    elif what == "tiny row":
+        L[701] *= np.float32(2.0**-119)
+    elif what == "tiny column":
+        R[:, 1503] *= np.float32(2.0**-119)
+    else:  # beside ordinary rows, all sums below 2^80
+        L[701] *= np.float32(2.0**-134)
+        R[:, 1503] *= np.float32(2.0**60)
+    got = []
+    assert any(x.startswith("zk_split_") for x in used(ctx, lambda: got.append(product(ctx, L, R, lt, rt))))
+    ref = L.astype(np.float64) @ R.astype(np.float64)
+    # Element (i, j) in units of |L_i| |R_j| / sqrt(k), its typical size; results
+    # below 2^-126 are themselves rounded to 2^-149.
+    unit = np.linalg.norm(L.astype(np.float64), axis=1)[:, None] * np.linalg.norm(R.astype(np.float64), axis=0) / np.sqrt(k)
+    e = np.maximum(np.abs(got[0] - ref) - 2.0**-149, 0.0) / unit
+    rms = [np.sqrt(np.mean(e * e, axis=axis)).max() for axis in (0, 1)]
+    print(f"[gpu] split gemm {what} {lt} {rt}: worst rms of a column {rms[0]:.1e}, of a row {rms[1]:.1e}", flush=True)
+    assert max(rms) <= 1e-6
+
+
 @pytest.mark.parametrize("rows", [12288, 12301])
 def test_split_gemm_network(ctx, rows):
     """Forward (both accumulator forms), data and weight gradients of a

@@ -2,7 +2,11 @@
 // split into three bf16 pieces (v_mfma_f32_32x32x16_bf16).
 //
 // x = h + m + l with h, m, l the successive bf16 roundings: 3 x 8 significant
-// bits hold all 24 bits of an fp32 value. A product keeps the six terms down
+// bits hold all 24 bits of an fp32 value, once the operands are scaled by 2^24:
+// the last bit of the smallest subnormal, 2^-149, is then a normal bf16 value. A
+// scaled value past the bf16 range or a sum past the fp32 range (operands from
+// 2^104, results from 2^80) comes out non-finite and is recomputed on the fp32
+// MFMAs. A product keeps the six terms down
 // to 2^-16 of the largest (h.h, h.m, m.h, h.l, m.m, l.h; the dropped ones lie
 // below 2^-26), accumulated in fp32, smallest first. Against float64 the sums
 // are closer than the fp32 MFMA's, because 16 products enter the accumulator
@@ -63,6 +67,10 @@ __device__ __forceinline__ Pieces split_pieces(const float (&x)[8]) {
 }
 
 constexpr int kSplitBK = 32;  // k-tile: two 16-wide MFMA steps
+// Of either operand before it is split: one multiplication per value, 0-4 %
+// of a case's time (returns of 98,304 rows 392 -> 410 us, two layers of 24,576
+// rows forward and backward 250 -> 253); sums in the ordinary range keep their bits.
+constexpr float kSplitScale = 0x1p24f;
 
 // LDS of one block in bytes: the B tile's pieces, double buffered.
 template <int CT>  // 32-wide column tiles of the block
@@ -253,6 +261,8 @@ __device__ __forceinline__ void split_body(char* __restrict__ smem, const GemmAr
         for (int c = 0; c < 8; ++c)
           if (k0 + split_k(s, g, c) >= K) braw[f][c] = 0.f;
       }
+#pragma unroll
+      for (int c = 0; c < 8; ++c) braw[f][c] *= kSplitScale;
       const Pieces q = split_pieces(braw[f]);
       char* d = base + ((n / 32) * 2 + s) * 3 * 1024 + slot(n & 31, g) * 16;
       *reinterpret_cast<bf16x8*>(d) = q.h;
@@ -266,7 +276,9 @@ __device__ __forceinline__ void split_body(char* __restrict__ smem, const GemmAr
   // rounding of one element but visible in a sum over a whole batch. So every
   // other strip (in rows, column blocks and split-K slices) accumulates -C.
   // (With ACC2 the small products never meet the large accumulator.)
-  float sgn = !ACC2 && (mt * WM + wm + nt + split) % 2 ? -1.f : 1.f;
+  const bool neg = !ACC2 && (mt * WM + wm + nt + split) % 2;
+  const float scale = neg ? -kSplitScale : kSplitScale;
+  float unscale = (neg ? -1.f : 1.f) / (kSplitScale * kSplitScale);
   constexpr int U = TN % 2 == 0 ? 2 : 1;  // column tiles whose MFMAs alternate
   floatx16 acc[TR][TN], lo[ACC2 ? TR : 1][ACC2 ? TN : 1];
 #pragma unroll
@@ -319,10 +331,8 @@ __device__ __forceinline__ void split_body(char* __restrict__ smem, const GemmAr
 #pragma unroll
           for (int c = 0; c < 8; ++c) rs[i] += araw[s][i][c];
         }
-        if constexpr (!ACC2) {
 #pragma unroll
-          for (int c = 0; c < 8; ++c) araw[s][i][c] *= sgn;
-        }
+        for (int c = 0; c < 8; ++c) araw[s][i][c] *= scale;
         const Pieces q = split_pieces(araw[s][i]);
         ah[i] = q.h, am[i] = q.m, al[i] = q.l;
       }
@@ -397,23 +407,19 @@ __device__ __forceinline__ void split_body(char* __restrict__ smem, const GemmAr
   load_y(0, 0);
 
   // Where the pieces do not hold the operands -- infinities (inf - inf), values
-  // that round to a bf16 infinity, or a strip so small that low pieces fall
-  // below the bf16 range -- the sums come out non-finite or tiny. Such a
-  // wavefront recomputes its strip with fp32 MFMAs straight from memory.
+  // that round to a bf16 infinity -- or a scaled sum overflows, the sums come
+  // out non-finite. Such a wavefront recomputes its strip with fp32 MFMAs
+  // straight from memory.
   {
-    float nan = 0.f, top = 0.f;
+    float nan = 0.f;
 #pragma unroll
     for (int i = 0; i < TR; ++i)
 #pragma unroll
       for (int j = 0; j < TN; ++j)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          nan = nan + acc[i][j][r] * 0.f;  // 0, or NaN once a sum is not finite
-          top = fmaxf(top, fabsf(acc[i][j][r]));
-        }
-    const bool redo = __any(nan != 0.f) || (__any(top > 0.f) && !__any(top >= 0x1p-80f));
-    if (redo) {
-      sgn = 1.f;
+        for (int r = 0; r < 16; ++r) nan = nan + acc[i][j][r] * 0.f;  // 0, or NaN once a sum is not finite
+    if (__any(nan != 0.f)) {
+      unscale = 1.f;
 #pragma unroll
       for (int i = 0; i < TR; ++i)
 #pragma unroll
@@ -462,7 +468,7 @@ __device__ __forceinline__ void split_body(char* __restrict__ smem, const GemmAr
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
           const int mm = min(mw + 32 * i + 4 * lg + 8 * (r / 4) + r % 4, p.M - 1);
-          C[(long long)mm * p.ldc + n] = f(ACC2 ? acc[i][j][r] : acc[i][j][r] * sgn, j, mm, n);
+          C[(long long)mm * p.ldc + n] = f(acc[i][j][r] * unscale, j, mm, n);
         }
       }
   };
@@ -478,7 +484,7 @@ __device__ __forceinline__ void split_body(char* __restrict__ smem, const GemmAr
 #pragma unroll
           for (int r = 0; r < 16; ++r)
             st[(4 * lg + 8 * (r / 4) + r % 4) * SPITCH + 32 * jj + li] =
-                  acc[i][SCOLS / 32 * h + jj][r] * sgn;
+                  acc[i][SCOLS / 32 * h + jj][r] * unscale;
 #pragma unroll
         for (int ps = 0; ps < SPASS; ++ps) {
           const int row = SROWS * ps + sr;
