@@ -1,0 +1,55 @@
+"""The GEMM planner on the CPU (plan_check.cpp around runtime.cpp): operands that
+a variant would not gather, split-K scratch, and which variants a size takes."""
+
+import os
+import shutil
+import subprocess
+
+import pytest
+
+from conftest import ROOT
+
+STORE, BIAS_N, BIAS_M, ELU_GRAD = range(4)
+
+
+@pytest.fixture(scope="module")
+def ask(tmp_path_factory):
+    rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
+    cxx = shutil.which("g++")
+    if not cxx or not os.path.isdir(f"{rocm}/include/hip"):
+        pytest.skip("no g++ or HIP headers")
+    exe = str(tmp_path_factory.mktemp("plan") / "plan_check")
+    subprocess.run([cxx, "-w", "-O1", "-std=c++17", "-D__HIP_PLATFORM_AMD__", f"-I{rocm}/include", f"-I{ROOT}/include",
+                    f"{ROOT}/tests/plan_check.cpp", "-o", exe, f"-L{rocm}/lib", f"-Wl,-rpath,{rocm}/lib", "-lamdhip64",
+                    "-ldl"], check=True)
+
+    def go(*lines):
+        text = "\n".join(" ".join(str(int(x) if isinstance(x, bool) else x) for x in line) for line in lines) + "\n"
+        return subprocess.run([exe], input=text, text=True, check=True, capture_output=True).stdout.splitlines()
+
+    return go
+
+
+def test_ungathered_operands_are_refused(ask):
+    """A variant that would read B (or A) in order although the problem gathers
+    it is refused; the gathers that the library uses are not."""
+    refused = [(24576, 256, 128, True, False, ELU_GRAD, 128, 256, False, True),   # three-piece, K-contiguous A
+               (24576, 256, 512, True, True, BIAS_N, 512, 512, False, True),      # three-piece forward
+               (300, 256, 512, True, True, BIAS_N, 512, 512, False, True),        # strips of a short minibatch
+               (4096, 512, 29, True, False, ELU_GRAD, 32, 512, False, True)]      # narrow K
+    taken = [(24576, 512, 124, True, True, BIAS_N, 124, 124, True, False),        # a shuffled minibatch's forward
+             (512, 124, 24576, False, False, STORE, 512, 124, False, True),       # and weight gradient
+             (300, 512, 128, True, True, BIAS_N, 128, 128, True, False),
+             (29, 128, 24576, False, False, STORE, 32, 128, False, True)]
+    assert ask(*[("plan", *p) for p in refused]) == ["refused"] * len(refused)
+    assert all(x != "refused" for x in ask(*[("plan", *p) for p in taken]))
+
+
+@pytest.mark.parametrize("m,n", [(512, 123), (512, 124), (512, 128), (256, 512), (128, 256), (256, 288), (512, 64),
+                                 (29, 128), (1, 128), (100, 33)])
+def test_split_k_scratch_covers_every_shorter_batch(ask, m, n):
+    """The scratch reserved for batches of up to K rows holds the partials of
+    any K' <= K, whatever variant K' takes (a shortfall would refuse the call)."""
+    for line in ask(*[("scratch", m, n, k) for k in (1, 40, 129, 384, 1000, 2400, 6145, 24577)]):
+        have, need = map(int, line.split())
+        assert have >= need

@@ -443,6 +443,16 @@ struct GemmPlan {
   unsigned gx = 0, gy = 0;
 };
 
+// Whether a variant honours the problem's permA / permB.
+static bool gathers(const GemmKernel& g, const GemmDesc& d) {
+  switch (g.kind) {
+    case G_SPLIT: return (!d.permA || d.a_kc) && (!d.permB || (!d.a_kc && !d.b_kc));
+    case G_NARROW_N:
+    case G_NARROW_K: return !d.permB;
+    default: return true;
+  }
+}
+
 static zl_status plan_gemm(zl_ctx* c, const GemmDesc& d, GemmPlan& P) {
   // float4 row loads need 16-byte aligned rows that cover the padded extent.
   const int a_ext = d.a_kc ? d.K : d.M;
@@ -458,8 +468,7 @@ static zl_status plan_gemm(zl_ctx* c, const GemmDesc& d, GemmPlan& P) {
   const bool vec_ok = g.kind == G_SPLIT ? kvec : P.vec;
   if (g.a_kc != d.a_kc || g.b_kc != d.b_kc || (g.vec && !vec_ok) || (g.need_vec_b && !(vb && plain)))
     return fail(c, ZL_ERR_INVALID, "GEMM variant %s does not match the operand layout", g.name);
-  if (g.kind == G_SPLIT && ((d.permA && !d.a_kc) || (d.permB && d.b_kc)))
-    return fail(c, ZL_ERR_INVALID, "GEMM variant %s gathers storage rows of A[M][K] and B[K][N] only", g.name);
+  if (!gathers(g, d)) return fail(c, ZL_ERR_INVALID, "GEMM variant %s does not gather these operands", g.name);
   if (strstr(g.name, "xk128") && (d.K > 128 || !plain))
     return fail(c, ZL_ERR_INVALID, "GEMM variant %s takes K <= 128 without split-K, row sums or gathers",
                 g.name);
