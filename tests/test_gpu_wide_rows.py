@@ -4,9 +4,10 @@ of short minibatches (zk_narrow_n1_v, zk_narrow_f22)."""
 
 import numpy as np
 import pytest
+import torch
 
 from oracle import zl_oracle as zo
-from zealot_amd import ops, synth
+from zealot_amd import DeviceBuffer, ops, synth
 from zealot_amd.rl import GpuMlp
 
 pytestmark = pytest.mark.gpu
@@ -19,6 +20,21 @@ def test_row_sum_exact_on_integers(ctx, m, n):
     out = ctx.alloc(m)
     ops.row_sum(ctx, out, ctx.to_device(x), m, n)
     assert np.array_equal(out.numpy(), x.sum(1, dtype=np.float64).astype(np.float32))
+
+
+def test_row_sum_of_two_billion_columns(ctx):
+    """A row whose last indices plus a block's stride lie past 2^31."""
+    n = 2**31 - 1000
+    x = torch.zeros(n, device="cuda")
+    x[0], x[n // 2], x[n - 1] = 1, 2, 4
+    torch.cuda.synchronize()
+    dx, out = DeviceBuffer(ctx, x.data_ptr(), 4 * n, (1, n), np.float32), ctx.alloc(1)
+    ops.row_sum(ctx, out, dx, 1, n)
+    dx.ptr = 0  # torch frees it
+    got = out.numpy()[0]
+    del x
+    torch.cuda.empty_cache()
+    assert got == 7
 
 
 @pytest.mark.parametrize("bad", [np.inf, -np.inf, np.nan])

@@ -676,9 +676,10 @@ __device__ void row_sum_wide_body(const RowSumArgs& p) {
   constexpr int T = kRowSumWideThreads, U = 8;
   const float* x = p.x + (long long)blockIdx.x * p.ldx;
   const int t = threadIdx.x;
+  const unsigned cols = (unsigned)p.cols;  // indices up to 2^31 + 8,191
   float s[U] = {};
-  int c = t;
-  for (; c + (U - 1) * T < p.cols; c += U * T) {
+  unsigned c = t;
+  for (; c + (U - 1) * T < cols; c += U * T) {
     float v[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) v[u] = x[c + u * T];
@@ -687,7 +688,7 @@ __device__ void row_sum_wide_body(const RowSumArgs& p) {
   }
 #pragma unroll
   for (int u = 0; u < U; ++u)
-    if (c + u * T < p.cols) s[u] += x[c + u * T];
+    if (c + u * T < cols) s[u] += x[c + u * T];
   float w = ((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7]));
   for (int o = 32; o > 0; o >>= 1) w += __shfl_xor(w, o);
   if ((t & 63) == 0) red[t >> 6] = w;
