@@ -3,6 +3,7 @@
 // touches a device.
 //
 //   plan M N K a_kc b_kc epi lda ldb permA permB   "<kernel> <slices>" or "refused"
+//   names                                           every kernel's name on one line
 //   scratch M N K                                   "<floats reserved for up to K rows> <most that any takes>"
 #include "../zealot_amd/csrc/runtime/runtime.cpp"
 
@@ -51,6 +52,9 @@ int main() {
         std::puts("refused");
       else
         std::printf("%s %d\n", kGemmTable[P.kid - K_GEMM_BASE].name, P.splits);
+    } else if (cmd == "names") {
+      for (int k = 0; k < K_GEMM_BASE + kGemmCount; ++k) std::printf("%s ", kernel_name(k));
+      std::puts("");
     } else {  // a weight gradient's scratch, reserved for K rows and used for any up to K
       int M, N, K;
       in >> M >> N >> K;

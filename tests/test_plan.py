@@ -53,3 +53,16 @@ def test_split_k_scratch_covers_every_shorter_batch(ask, m, n):
     for line in ask(*[("scratch", m, n, k) for k in (1, 40, 129, 384, 1000, 2400, 6145, 24577)]):
         have, need = map(int, line.split())
         assert have >= need
+
+
+def test_bench_counts_every_gemm_kernel(ask):
+    """The layer GEMM time and FLOPs that bench.py reports cover every GEMM
+    kernel of the table and the fixed kernels that contain one, and no other."""
+    import bench
+
+    names = ask(("names",))[0].split()
+    fixed = {x for x in names[:names.index("zk_policy_pack") + 1]
+             if x.startswith(("zk_gemm_bwd", "zk_split_bwd", "zk_head_fwd"))}
+    table = set(names[names.index("zk_policy_pack") + 1:])
+    assert {"zk_split_bwd", "zk_head_fwd"} <= fixed and {"zk_split_ak_bn_dg", "zk_narrow_f22"} <= table
+    assert {x for x in names if bench.is_layer_gemm(x)} == fixed | table
