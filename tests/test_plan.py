@@ -55,6 +55,16 @@ def test_split_k_scratch_covers_every_shorter_batch(ask, m, n):
         assert have >= need
 
 
+@pytest.mark.parametrize("rows", [3072, 4096, 4608, 5376, 6016, 24576])
+@pytest.mark.parametrize("n,k", [(128, 128), (128, 64), (256, 128)])
+def test_backward_of_a_layer_is_one_launch(ask, rows, n, k):
+    """run_gemm_bwd merges a layer's weight and data gradients where both take
+    the three-piece variants."""
+    got = ask(("plan", rows, n, k, True, False, ELU_GRAD, k, n, False, False),
+              ("plan", k, n, rows, False, False, STORE, k, n, False, False))
+    assert [x.split()[0] for x in got] == ["zk_split_ak_bn_dg", "zk_split_am_bn"]
+
+
 def test_bench_counts_every_gemm_kernel(ask):
     """The layer GEMM time and FLOPs that bench.py reports cover every GEMM
     kernel of the table and the fixed kernels that contain one, and no other."""

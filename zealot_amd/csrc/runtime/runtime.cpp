@@ -201,7 +201,10 @@ static int pick_split(const zl_ctx* c, int M, int N, int K, int lay, int epi, bo
       epi == zk::kEpiStore ? std::min(cdiv(256, tiles), max_slices(K / 32)) : 1;
   long long least = 48;
   if (lay == L_AK_BK && epi != zk::kEpiStore) least = M <= 2048 ? LLONG_MAX : K <= 64 ? 192 : 64;
-  if (lay == L_AK_BN && epi != zk::kEpiEluGrad) least = 256;
+  // Data gradients share a launch with their layer's weight gradient where both
+  // are three-piece (us per minibatch of 48-128-128-8 nets, 42 tiles: 75, apart 87;
+  // of 64-256-128-64-12 nets, 24 tiles: 102 / 109, 16 tiles: 98 / 95).
+  if (lay == L_AK_BN) least = epi == zk::kEpiEluGrad ? 24 : 256;
   if (tiles * slices < least) return -1;
   switch (lay) {
     case L_AK_BK:
