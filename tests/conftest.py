@@ -38,3 +38,19 @@ def ulp_diff(a, b) -> int:
     a = np.where(a < 0, -(a & 0x7FFFFFFF), a)
     b = np.where(b < 0, -(b & 0x7FFFFFFF), b)
     return int(np.max(np.abs(a - b))) if a.size else 0
+
+
+def launches(ctx, fn):
+    """Names of the kernels that fn launches, in order."""
+    import ctypes as C
+
+    ctx.check(ctx.lib.zl_timing_begin(ctx.h, b"*"))
+    fn()
+    n = C.c_longlong()
+    ctx.check(ctx.lib.zl_timing_end(ctx.h, None, C.byref(n), None))
+    names = []
+    for i in range(n.value):
+        name = C.c_char_p()
+        ctx.check(ctx.lib.zl_timing_launch(ctx.h, i, C.byref(name), None, None, None))
+        names.append(name.value.decode())
+    return names

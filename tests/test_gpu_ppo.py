@@ -17,7 +17,7 @@ import numpy as np
 import pytest
 
 import np_ref
-from conftest import rel_amax
+from conftest import launches, rel_amax
 from oracle import zl_oracle as zo
 from zealot_amd import Context, ZealotError, synth
 from zealot_amd.rl import DeviceBatch, GpuActorCritic, PpoConfig
@@ -298,10 +298,9 @@ def test_head_forward_fused_matches_separate(ctx, n, shuffled):
 
 @pytest.mark.parametrize("shuffled", [False, True])
 def test_backward_merged_matches_separate(ctx, shuffled):
-    """A layer's weight- and data-gradient GEMMs as one zk_gemm_bwd_* launch
-    against the same GEMMs as two launches (ZL_MERGED_BWD=0): the 512 -> 256
-    layer takes the 128 x 128 weight-gradient form, the 256 -> 128 layer the
-    64 x 128 one, and both runs are bit-identical — the minibatch gradients
+    """A layer's weight- and data-gradient GEMMs as one zk_split_bwd launch (the
+    512 -> 256 and the 256 -> 128 layer) against the same GEMMs as two launches
+    (ZL_MERGED_BWD=0): both runs are bit-identical — the minibatch gradients
     and a whole update (2 epochs x 2 minibatches of 3,072 rows)."""
     ad, cd = [64, 512, 256, 128, 12], [64, 512, 256, 128, 1]
     n = 6144
@@ -326,7 +325,9 @@ def test_backward_merged_matches_separate(ctx, shuffled):
         perm = cx.to_device(order) if shuffled else None
         gac = GpuActorCritic(cx, ad, cd, n)
         gac.set_params(actor, critic, log_std, 1e-3)
-        grads = gac.minibatch_grads(db, PpoConfig(entropy_coef=0.01), 0, n, perm=perm)
+        grads = []
+        names = launches(cx, lambda: grads.extend(gac.minibatch_grads(db, PpoConfig(entropy_coef=0.01), 0, n, perm=perm)))
+        assert names.count("zk_split_bwd") == (2 if merged else 0), names
         gac.update(db, PpoConfig(epochs=2, minibatches=2))
         out.append((grads, gac.get_params()))
         gac.close()

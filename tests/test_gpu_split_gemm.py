@@ -8,6 +8,7 @@ import os
 import numpy as np
 import pytest
 
+from conftest import launches as used
 from zealot_amd import ops, synth
 
 pytestmark = pytest.mark.gpu
@@ -33,22 +34,6 @@ def product(ctx, L, R, lt, rt):
     dr = ctx.to_device(np.ascontiguousarray(R.T if rt else R))
     ops.gemm(ctx, out, dl, lt, dr, rt, m, n, k)
     return out.numpy()
-
-
-def used(ctx, fn):
-    """Names of the GEMM kernels that fn launches."""
-    import ctypes as C
-
-    ctx.check(ctx.lib.zl_timing_begin(ctx.h, b"*"))
-    fn()
-    n = C.c_longlong()
-    ctx.check(ctx.lib.zl_timing_end(ctx.h, None, C.byref(n), None))
-    names = []
-    for i in range(n.value):
-        name = C.c_char_p()
-        ctx.check(ctx.lib.zl_timing_launch(ctx.h, i, C.byref(name), None, None, None))
-        names.append(name.value.decode())
-    return names
 
 
 # (m, n, k, lhs_t, rhs_t): whole tiles; one past and one short of a tile in each

@@ -71,8 +71,7 @@ def test_bench_counts_every_gemm_kernel(ask):
     import bench
 
     names = ask(("names",))[0].split()
-    fixed = {x for x in names[:names.index("zk_policy_pack") + 1]
-             if x.startswith(("zk_gemm_bwd", "zk_split_bwd", "zk_head_fwd"))}
+    fixed = {x for x in names[:names.index("zk_policy_pack") + 1] if x.startswith(("zk_split_bwd", "zk_head_fwd"))}
     table = set(names[names.index("zk_policy_pack") + 1:])
     assert {"zk_split_bwd", "zk_head_fwd"} <= fixed and {"zk_split_ak_bn_dg", "zk_narrow_f22"} <= table
     assert {x for x in names if bench.is_layer_gemm(x)} == fixed | table

@@ -46,10 +46,6 @@ enum KernelId : int {
   K_SUMSQ_MULTI,
   K_CLIP_SCALE,
   K_ADAM_MULTI,
-  K_GEMM_BWD_128,
-  K_GEMM_BWD_64,
-  K_GEMM_BWD_128_D128,
-  K_GEMM_BWD_64_D128,
   K_SPLIT_BWD,
   K_HEAD_FWD,
   K_HEAD_FWD_X,
@@ -173,8 +169,8 @@ struct zl_ctx {
   // off) and the block count their row slices aim at (ZL_NARROW_TARGET).
   bool narrow = true;
   int narrow_target = 256;
-  // A layer's weight- and data-gradient GEMMs as one launch where a merged
-  // kernel covers their variants (ZL_MERGED_BWD=0 runs them as two).
+  // A layer's weight- and data-gradient GEMMs as one launch where zk_split_bwd
+  // covers their variants (ZL_MERGED_BWD=0 runs them as two).
   bool merged_bwd = true;
   // Forwards of up to kPolicyFusedRows rows (a rollout step) as one zk_policy
   // launch where the nets fit it (ZL_POLICY_FUSED=0 keeps the layer GEMMs).
@@ -275,9 +271,9 @@ zl_status run_gemm(zl_ctx* c, const GemmDesc& d);
 // launches); problems that split K over slices need caller scratch when n > 1.
 zl_status run_gemm_batch(zl_ctx* c, const GemmDesc* d, int n);
 // A layer's backward: the weight-gradient batch w and the data-gradient
-// batch d (nd may be 0), as one zk_gemm_bwd_* launch when both are single
-// exact-fit launches of the variants it covers, else as run_gemm_batch(w)
-// then run_gemm_batch(d).
+// batch d (nd may be 0), as one zk_split_bwd launch when both are single
+// launches of the three-piece variants, else as run_gemm_batch(w) then
+// run_gemm_batch(d).
 zl_status run_gemm_bwd(zl_ctx* c, const GemmDesc* w, int nw, const GemmDesc* d, int nd);
 // Block layout of zk_reduce_all over `segs` (fills lanes / blk0 / nqb / nrb);
 // returns the block count (= number of sum-of-squares partials).

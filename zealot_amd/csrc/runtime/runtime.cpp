@@ -23,7 +23,7 @@ const char* const kFixedNames[K_GEMM_BASE] = {
     "zk_norm_apply",
     "zk_norm_stats",    "zk_norm_merge",  "zk_norm_commit", "zk_sample_g32",  "zk_sample_g64",
     "zk_stage",         "zk_sumsq_multi", "zk_clip_scale",  "zk_adam_multi",
-    "zk_gemm_bwd_128x128_dg_x", "zk_gemm_bwd_64x128_dg_x", "zk_gemm_bwd_128x128_dg128_x", "zk_gemm_bwd_64x128_dg128_x", "zk_split_bwd", "zk_head_fwd", "zk_head_fwd_x",
+    "zk_split_bwd", "zk_head_fwd", "zk_head_fwd_x",
     "zk_policy",        "zk_transpose",   "zk_policy_pack",
 };
 
@@ -39,9 +39,7 @@ const GemmKernel kGemmTable[] = {
     {"zk_gemm_ak_bk_96x128x32_w24_x", true, true, 96, 128, 32, 512, true},
     {"zk_gemm_ak_bk_128x128x32_w24", true, true, 128, 128, 32, 512, true},
     {"zk_gemm_ak_bk_128x128x32_w24_x", true, true, 128, 128, 32, 512, true},
-    {"zk_gemm_ak_bn_96x128x32_w24_dg_x", true, false, 96, 128, 32, 512, true},
     {"zk_gemm_ak_bn_128x128x32_w24_dg", true, false, 128, 128, 32, 512, true},
-    {"zk_gemm_ak_bn_128x128x32_w24_dg_x", true, false, 128, 128, 32, 512, true},
     {"zk_gemm_am_bn_128x128x32_w24_x", false, false, 128, 128, 32, 512, true},
     {"zk_gemm_am_bn_64x128x32_w24_x", false, false, 64, 128, 32, 512, true},
     {"zk_gemm_am_bn_64x128x32_w24", false, false, 64, 128, 32, 512, true},
@@ -726,26 +724,8 @@ zl_status run_gemm_bwd(zl_ctx* c, const GemmDesc* w, int nw, const GemmDesc* d, 
     zl_status s = plan_batch(c, w, nw, W, ow);
     if (s) return s;
     if (ow && W.nl > 0 && (s = plan_batch(c, d, nd, D, od))) return s;
-    int mk = -1;
-    if (ow && od && W.nl > 0 && D.nl > 0 && D.kid == gemm_id("zk_gemm_ak_bn_96x128x32_w24_dg_x")) {
-      if (W.kid == gemm_id("zk_gemm_am_bn_128x128x32_w24_x"))
-        mk = K_GEMM_BWD_128;
-      else if (W.kid == gemm_id("zk_gemm_am_bn_64x128x32_w24_x"))
-        mk = K_GEMM_BWD_64;
-    }
-    if (ow && od && W.nl > 0 && D.nl > 0 && D.kid == gemm_id("zk_gemm_ak_bn_128x128x32_w24_dg_x")) {
-      if (W.kid == gemm_id("zk_gemm_am_bn_128x128x32_w24_x"))
-        mk = K_GEMM_BWD_128_D128;
-      else if (W.kid == gemm_id("zk_gemm_am_bn_64x128x32_w24_x"))
-        mk = K_GEMM_BWD_64_D128;
-    }
-    unsigned threads = 512;
     if (ow && od && W.nl > 0 && D.nl > 0 && D.kid == gemm_id("zk_split_ak_bn_dg") &&
         W.kid == gemm_id("zk_split_am_bn")) {
-      mk = K_SPLIT_BWD;
-      threads = 256;
-    }
-    if (mk >= 0) {
       zk::GemmPair a{};
       a.w = W.B;
       a.d = D.B;
@@ -753,7 +733,7 @@ zl_status run_gemm_bwd(zl_ctx* c, const GemmDesc* w, int nw, const GemmDesc* d, 
       const long long blocks = (long long)W.gx + D.gx;
       c->pending_flops = W.flops + D.flops;
       c->pending_shape = {D.live[0]->M, D.live[0]->N, D.live[0]->K, W.P[0].splits};
-      s = launch(c, mk, (unsigned)blocks, 1, 1, a, 0, threads);
+      s = launch(c, K_SPLIT_BWD, (unsigned)blocks, 1, 1, a, 0, W.threads);
       if (!s) s = finish_batch(c, W);
       return s ? s : finish_batch(c, D);
     }
