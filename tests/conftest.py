@@ -40,8 +40,9 @@ def ulp_diff(a, b) -> int:
     return int(np.max(np.abs(a - b))) if a.size else 0
 
 
-def launches(ctx, fn):
-    """Names of the kernels that fn launches, in order."""
+def launches(ctx, fn, shapes=None):
+    """Names of the kernels that fn launches, in order; (M, N, K, slices) of
+    each GEMM launch (zeros of the others) appended to shapes."""
     import ctypes as C
 
     ctx.check(ctx.lib.zl_timing_begin(ctx.h, b"*"))
@@ -50,7 +51,9 @@ def launches(ctx, fn):
     ctx.check(ctx.lib.zl_timing_end(ctx.h, None, C.byref(n), None))
     names = []
     for i in range(n.value):
-        name = C.c_char_p()
-        ctx.check(ctx.lib.zl_timing_launch(ctx.h, i, C.byref(name), None, None, None))
+        name, shape = C.c_char_p(), (C.c_int * 4)()
+        ctx.check(ctx.lib.zl_timing_launch(ctx.h, i, C.byref(name), None, None, shape))
         names.append(name.value.decode())
+        if shapes is not None:
+            shapes.append(tuple(shape))
     return names

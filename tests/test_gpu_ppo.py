@@ -283,7 +283,9 @@ def test_head_forward_fused_matches_separate(ctx, n, shuffled):
         finally:
             os.environ.pop("ZL_FUSED_HEAD", None)
         gac.set_params(actor, critic, log_std, 1e-3)
-        out.append(gac.minibatch_grads(db, PpoConfig(entropy_coef=0.01), 0, n, perm=perm))
+        names = launches(ctx, lambda: out.append(gac.minibatch_grads(db, PpoConfig(entropy_coef=0.01), 0, n, perm=perm)))
+        want = "zk_head" if not fused_fwd else "zk_head_fwd_x" if n % 64 == 0 else "zk_head_fwd"
+        assert [x for x in names if x.startswith("zk_head")] == [want], names
         gac.close()
     (fa, fc, fl, fs), (sa, sc, sl, ss) = out
     assert np.array_equal(fa, sa) and np.array_equal(fl, sl)
