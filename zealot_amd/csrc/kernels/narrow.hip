@@ -333,7 +333,13 @@ __device__ __forceinline__ void narrow_f_body(const GemmArgs& p, float (&red)[kN
   constexpr int P = 4;  // chunks whose loads are issued together
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
   const int lr = lane & 15, lg = lane >> 4;
-  const int n0 = blockIdx.x * 16 * NT, m0 = blockIdx.y * 16 * MT;
+  // Workgroups reach the 8 XCDs round robin: each XCD takes a contiguous run of
+  // tiles, rows fastest, so that its L2 holds an eighth of B and not all of it,
+  // which would evict the next launch's operands (layers 265 -> 512 -> 256 over
+  // 1,500 columns: 59 -> 42 us, 47 on the 64 x 64 tiles).
+  const int g = blockIdx.x + gridDim.x * blockIdx.y, all = gridDim.x * gridDim.y, x = g % 8;
+  const int tile = x * (all / 8) + min(x, all % 8) + g / 8;
+  const int n0 = tile / gridDim.y * 16 * NT, m0 = tile % gridDim.y * 16 * MT;
   if (n0 >= p.N || m0 >= p.M) return;  // uniform: a paired problem's larger grid
   const float* b[NT];
 #pragma unroll
