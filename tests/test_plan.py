@@ -65,6 +65,15 @@ def test_backward_of_a_layer_is_one_launch(ask, rows, n, k):
     assert [x.split()[0] for x in got] == ["zk_split_ak_bn_dg", "zk_split_am_bn"]
 
 
+@pytest.mark.parametrize("m,n,k,want", [(256, 1000, 264, "zk_narrow_f22"), (256, 1500, 264, "zk_gemm_ak_bn_64x64x32_w22"),
+                                        (512, 1000, 520, "zk_gemm_ak_bn_64x64x32_w22"), (512, 1000, 512, "zk_narrow_f22"),
+                                        (512, 1000, 265, "zk_narrow_f22"), (512, 1500, 265, "zk_gemm_ak_bn_64x64x32_w22_s")])
+def test_feature_major_layers_with_few_tiles(ask, m, n, k, want):
+    """Where the K-splitting kernel measured faster than the 64 x 64 tiles: two
+    tiles per CU, one where only the 64 x 64 tiles read A as float4 rows."""
+    assert ask(("plan", m, n, k, True, False, BIAS_M, k, n, False, False))[0].split()[0] == want
+
+
 def test_bench_counts_every_gemm_kernel(ask):
     """The layer GEMM time and FLOPs that bench.py reports cover every GEMM
     kernel of the table and the fixed kernels that contain one, and no other."""
