@@ -74,6 +74,16 @@ def test_feature_major_layers_with_few_tiles(ask, m, n, k, want):
     assert ask(("plan", m, n, k, True, False, BIAS_M, k, n, False, False))[0].split()[0] == want
 
 
+@pytest.mark.parametrize("m,n,k,want", [(512, 8192, 64, False), (512, 10_000, 64, False), (256, 24_576, 64, True),
+                                        (256, 24_576, 36, False), (512, 16_384, 36, True), (512, 10_000, 256, False),
+                                        (512, 8192, 264, True), (512, 8193, 265, True), (512, 24_576, 128, True)])
+def test_feature_major_layers_on_three_pieces(ask, m, n, k, want):
+    """From 256 tiles of 128 x 128 on, with short reductions from 384 or 512, as
+    measured against the fp32 tiles."""
+    got = ask(("plan", m, n, k, True, False, BIAS_M, k, n, False, False))[0]
+    assert got.startswith("zk_split_ak_bn") == want, got
+
+
 def test_bench_counts_every_gemm_kernel(ask):
     """The layer GEMM time and FLOPs that bench.py reports cover every GEMM
     kernel of the table and the fixed kernels that contain one, and no other."""

@@ -190,7 +190,8 @@ inline long long max_slices(long long kt) { return std::max({1LL, kt / 8, std::m
 // 24,576 222 / 151; input-layer weight gradient 512 x 128 x 24,576 63 / 48.
 // Feature-major products (L_AK_BN without ELU'), one problem: 128 x 24,576 x
 // 256 26 / 29, 256 x 24,576 x 512 75 / 60. Narrow or half-empty tiles keep fp32.
-static int pick_split(const zl_ctx* c, int M, int N, int K, int lay, int epi, bool kvec) {
+// vec, kvec: as in pick_gemm.
+static int pick_split(const zl_ctx* c, int M, int N, int K, int lay, int epi, bool vec, bool kvec) {
   if (!c || !c->split_gemm || lay == L_AM_BK) return -1;
   const long long tiles = cdiv(M, 128) * cdiv(N, 128);
   if (2LL * M * N < tiles * 128 * 128) return -1;
@@ -202,7 +203,11 @@ static int pick_split(const zl_ctx* c, int M, int N, int K, int lay, int epi, bo
   // Data gradients share a launch with their layer's weight gradient where both
   // are three-piece (us per minibatch of 48-128-128-8 nets, 42 tiles: 75, apart 87;
   // of 64-256-128-64-12 nets, 24 tiles: 102 / 109, 16 tiles: 98 / 95).
-  if (lay == L_AK_BN) least = epi == zk::kEpiEluGrad ? 24 : 256;
+  // Other feature-major products, by K where the fp32 tiles read float4 rows
+  // (fp32 / three-piece, us, 256 tiles and 384): 36 13.2 / 17.7, 19.0 / 20.1; 64
+  // 13.2 / 17.2, 20.3 / 19.8; 128 19.3 / 20.6, 27.5 / 25.1; 256 28.3 / 27.9, 39.4 /
+  // 35.4 (34.0 / 34.7 at 316 tiles).
+  if (lay == L_AK_BN) least = epi == zk::kEpiEluGrad ? 24 : !vec || K > 256 ? 256 : K < 64 ? 512 : 384;
   if (tiles * slices < least) return -1;
   switch (lay) {
     case L_AK_BK:
@@ -227,7 +232,7 @@ int pick_gemm(const zl_ctx* c, int M, int N, int K, bool a_kc, bool b_kc, bool v
   // Narrow and small-K shapes keep their own kernels.
   const GemmKernel& g = kGemmTable[fp32 - K_GEMM_BASE];
   if (g.kind != G_TILED || strstr(g.name, "xk128")) return fp32;
-  const int split = pick_split(c, M, N, K, lay, epi, kvec);
+  const int split = pick_split(c, M, N, K, lay, epi, vec, kvec);
   return split >= 0 ? split : fp32;
 }
 
@@ -421,7 +426,7 @@ size_t gemm_ws_floats(const zl_ctx* c, int M, int N, int K, bool a_kc, bool b_kc
       s = std::max(s, std::min(cdiv(target, cdiv(M, g.bm) * cdiv(N, g.bn)), max_slices(kt)));
     }
   };
-  const int split = pick_split(c, M, N, K, lay, epi, true);
+  const int split = pick_split(c, M, N, K, lay, epi, false, true);  // the form with the lower threshold
   if (split >= 0) limit(split);
   for (bool vec : {true, false}) limit(pick_fp32(c, M, N, K, a_kc, b_kc, vec, epi, false));
   return s <= 1 ? 0 : (size_t)s * M * N + (size_t)s * M;
