@@ -3,6 +3,7 @@
 // touches a device.
 //
 //   plan M N K a_kc b_kc epi lda ldb permA permB   "<kernel> <slices>" or "refused"
+//   apart (the same)                                of a product whose partials a launch of its own sums
 //   names                                           every kernel's name on one line
 //   scratch M N K                                   "<floats reserved for up to K rows> <most that any takes>"
 #include "../zealot_amd/csrc/runtime/runtime.cpp"
@@ -18,7 +19,7 @@ void noalloc_release(zl_ctx*) {}
 using namespace zl;
 
 static zl_status plan(zl_ctx& c, int M, int N, int K, bool a_kc, bool b_kc, int epi, int lda, int ldb, bool pa, bool pb,
-                      GemmPlan& P) {
+                      bool apart, GemmPlan& P) {
   alignas(16) static float mem[4];
   static int perm[4];
   GemmDesc d;
@@ -35,6 +36,8 @@ static zl_status plan(zl_ctx& c, int M, int N, int K, bool a_kc, bool b_kc, int 
   d.epi = epi;
   d.permA = pa ? perm : nullptr;
   d.permB = pb ? perm : nullptr;
+  zk::ReduceSeg seg;
+  d.seg_out = apart ? nullptr : &seg;
   return plan_gemm(&c, d, P);
 }
 
@@ -44,11 +47,11 @@ int main() {
   while (std::getline(std::cin, line)) {
     std::istringstream in(line);
     in >> cmd;
-    if (cmd == "plan") {
+    if (cmd == "plan" || cmd == "apart") {
       int M, N, K, a, b, epi, lda, ldb, pa, pb;
       in >> M >> N >> K >> a >> b >> epi >> lda >> ldb >> pa >> pb;
       GemmPlan P;
-      if (plan(c, M, N, K, a, b, epi, lda, ldb, pa, pb, P))
+      if (plan(c, M, N, K, a, b, epi, lda, ldb, pa, pb, cmd == "apart", P))
         std::puts("refused");
       else
         std::printf("%s %d\n", kGemmTable[P.kid - K_GEMM_BASE].name, P.splits);
@@ -60,11 +63,11 @@ int main() {
       in >> M >> N >> K;
       size_t most = 0;
       for (int k = 1; k <= K; ++k)
-        for (int odd = 0; odd < 2; ++odd) {
+        for (int form = 0; form < 4; ++form) {
           GemmPlan P;
-          const int pad = odd ? 1 : 0;  // rows that are not float4-aligned
+          const int pad = form & 1;  // rows that are not float4-aligned
           if (plan(c, M, N, k, false, false, zk::kEpiStore, (int)round_up(M, 4) + pad, (int)round_up(N, 4) + pad, false,
-                   false, P))
+                   false, form & 2, P))
             continue;
           if (P.splits > 1) most = std::max(most, (size_t)P.splits * M * N + (size_t)P.splits * M);
         }

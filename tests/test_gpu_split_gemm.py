@@ -39,12 +39,12 @@ def product(ctx, L, R, lt, rt):
 # (m, n, k, lhs_t, rhs_t, variant): whole tiles; one past and one short of a tile
 # in each extent; K tails of 1, 31 and one k-tile; K not a multiple of 4 (element
 # loads); deep K with slices whose last one holds the tail.
-CASES = [(12288, 128, 32, False, True, "ak_bk"), (12289, 127, 33, False, True, "ak_bk_s"),
-         (8191, 257, 96, False, True, "ak_bk"), (12300, 130, 1, False, True, "ak_bk_s"),
+CASES = [(32768, 128, 32, False, True, "ak_bk"), (49153, 127, 33, False, True, "ak_bk_s"),
+         (8191, 257, 96, False, True, "ak_bk"), (49170, 250, 1, False, True, "ak_bk_s"),
          (6200, 256, 123, False, True, "ak_bk_s"), (256, 300, 8193, False, True, "ak_bk_s"),
          (250, 24577, 516, False, False, "ak_bn"), (384, 11000, 261, False, False, "ak_bn_s"),
          (255, 16500, 200, True, False, "am_bn"), (193, 513, 24577, True, False, "am_bn"),
-         (128, 256, 6144, True, False, "am_bn")]
+         (256, 512, 6144, True, False, "am_bn")]
 
 
 def as_exact_as_fp32(got, fp32, ref, tag):

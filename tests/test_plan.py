@@ -84,6 +84,21 @@ def test_feature_major_layers_on_three_pieces(ask, m, n, k, want):
     assert got.startswith("zk_split_ak_bn") == want, got
 
 
+@pytest.mark.parametrize("m,n,k,a,b,want", [(1500, 512, 256, 1, 0, "zk_gemm_ak_bn_64x64x32_w22 1"),
+                                            (16_384, 64, 288, 1, 1, "zk_gemm_ak_bk_64x64x32_w22 1"),
+                                            (128, 16_384, 256, 0, 0, "zk_gemm_am_bn_64x128x32_w24_x 1"),
+                                            (512, 512, 384, 0, 0, "zk_split_am_bn 6"),
+                                            (10_000, 512, 64, 1, 0, "zk_split_ak_bn 1"),
+                                            (256, 512, 24_576, 1, 1, "zk_split_ak_bk 32"),
+                                            (512, 24_576, 256, 0, 0, "zk_split_am_bn 1")])
+def test_products_summed_apart(ask, m, n, k, a, b, want):
+    """Products whose split-K partials take a launch of their own: few slices and
+    fp32 tiles where that launch and the traffic cost more than they save. (The
+    first three measured 10.2, 10.6 and 15.1 us, 15.4, 20.1 and 25.7 as a minibatch
+    runs them.)"""
+    assert ask(("apart", m, n, k, a, b, STORE, k if a else m, k if b else n, False, False)) == [want]
+
+
 def test_bench_counts_every_gemm_kernel(ask):
     """The layer GEMM time and FLOPs that bench.py reports cover every GEMM
     kernel of the table and the fixed kernels that contain one, and no other."""

@@ -260,9 +260,11 @@ struct GemmDesc {
 // vec_b: B alone can be read as float4 rows and the problem has no split-K,
 // row sums or gathers (the small-K variants may then take it).
 // kvec: every K-contiguous operand can be read as float4 rows (the three-piece
-// variants read the others by elements).
+// variants read the others by elements). fp32_only: no three-piece variant.
+// apart: split-K partials are summed by a launch of their own.
 int pick_gemm(const zl_ctx* c, int M, int N, int K, bool a_kc, bool b_kc, bool vec = true,
-              int epi = zk::kEpiStore, bool vec_b = false, bool kvec = true, bool fp32_only = false);
+              int epi = zk::kEpiStore, bool vec_b = false, bool kvec = true, bool fp32_only = false,
+              bool apart = false);
 int gemm_splits(const zl_ctx* c, int M, int N, int K, bool a_kc, bool b_kc, int epi,
                 bool vec = true);
 size_t gemm_ws_floats(const zl_ctx* c, int M, int N, int K, bool a_kc, bool b_kc, int epi);

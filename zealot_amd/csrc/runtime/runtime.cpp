@@ -203,11 +203,12 @@ static int pick_split(const zl_ctx* c, int M, int N, int K, int lay, int epi, bo
   // Data gradients share a launch with their layer's weight gradient where both
   // are three-piece (us per minibatch of 48-128-128-8 nets, 42 tiles: 75, apart 87;
   // of 64-256-128-64-12 nets, 24 tiles: 102 / 109, 16 tiles: 98 / 95).
-  // Other feature-major products, by K where the fp32 tiles read float4 rows
+  // Feature-major layers, by K where the fp32 tiles read float4 rows
   // (fp32 / three-piece, us, 256 tiles and 384): 36 13.2 / 17.7, 19.0 / 20.1; 64
   // 13.2 / 17.2, 20.3 / 19.8; 128 19.3 / 20.6, 27.5 / 25.1; 256 28.3 / 27.9, 39.4 /
   // 35.4 (34.0 / 34.7 at 316 tiles).
-  if (lay == L_AK_BN) least = epi == zk::kEpiEluGrad ? 24 : !vec || K > 256 ? 256 : K < 64 ? 512 : 384;
+  if (lay == L_AK_BN)
+    least = epi == zk::kEpiEluGrad ? 24 : epi == zk::kEpiStore || !vec || K > 256 ? 256 : K < 64 ? 512 : 384;
   if (tiles * slices < least) return -1;
   switch (lay) {
     case L_AK_BK:
@@ -223,9 +224,67 @@ static int pick_split(const zl_ctx* c, int M, int N, int K, int lay, int epi, bo
 
 static int pick_fp32(const zl_ctx* c, int M, int N, int K, bool a_kc, bool b_kc, bool vec, int epi,
                      bool vec_b);
+static int narrow_rows_per_slice(const zl_ctx* c, int N, int K, int epi);
+
+// Time, us, of a product without epilogue in `splits` slices whose partials a
+// launch of their own sums (less the launch itself, the same for any choice):
+// the k-tiles of a slice in series, more of them where blocks share a CU, the
+// second launch, its traffic, and its slices one by one where float4 quads would
+// cross rows of odd products. Constants fitted to 2,900 launches of 24 to 512 x
+// 384 to 24,576 x 12 to 24,576 in the three layouts. Of the faster of fp32 in
+// slices of eight k-tiles, in slices of two, and three-piece, the choice by it
+// loses 0.2 % in the mean and 18 % at worst. Always slices of two lost up to 54 %
+// (1,500 x 512 x 256 15.4 vs 10.2 us), three-piece wherever a minibatch takes it up
+// to 89 % (16,384 x 64 x 288 20.1 vs 10.6 us), slices of eight 38 % in the mean (512 x
+// 512 x 384 29.1 vs 14.5 us).
+static double apart_us(const GemmKernel& g, int M, int N, int K, int splits) {
+  const bool three = g.kind == G_SPLIT;
+  double kt_us;  // of one k-tile of a block
+  if (three)
+    kt_us = (g.a_kc || g.b_kc) && !g.vec ? 2.7 : g.a_kc ? 1.55 : 1.75;
+  else if (!g.vec)
+    kt_us = g.bn == 64 ? 2.0 : 1.6;
+  else
+    kt_us = g.bk == 32 ? std::max(0.7, 0.2 + 2.1 * g.bm * g.bn / (128.0 * 128.0)) : 0.54;
+  const double per_cu = cdiv(M, g.bm) * cdiv(N, g.bn) * splits / 256.0, mn = (double)M * N;
+  const double waves = per_cu <= 1.0 ? 1.0 : std::max(per_cu, three ? 1.1 : g.threads == 512 ? 1.8 : 1.4);
+  double us = waves * cdiv(cdiv(K, g.bk), splits) * kt_us + (three ? 0.1e-6 * splits * mn : 0.0);
+  if (splits > 1) us += 3.8 + 1.6e-6 * splits * mn + ((long long)M * N % 4 ? 0.3 * splits : 0.0);
+  return us;
+}
+
+// Split-K slices of a variant. apart: a launch of their own sums the partials
+// (else they wait for the all-layer reduction).
+static int slices_of(const zl_ctx* c, const GemmKernel& g, int M, int N, int K, int epi, bool apart) {
+  if (g.kind == G_NARROW_M) return (int)cdiv(std::max(K, 1), narrow_rows_per_slice(c, N, K, epi));
+  if (!is_tiled(g.kind)) return 1;
+  if (epi != zk::kEpiStore) return 1;
+  const long long tiles = cdiv(M, g.bm) * cdiv(N, g.bn);
+  const long long kt = cdiv(K, g.bk);
+  auto whole = [&](long long s) {
+    s = std::max<long long>(1, std::min(s, kt));
+    return (int)cdiv(kt, cdiv(kt, s));
+  };
+  if (c && c->force_splits > 0) return whole(c->force_splits);
+  // Deep-K, few-tile shapes (the weight gradients, K = batch rows) would
+  // leave most CUs idle: slice K so the grid reaches the split-K target
+  // (256 = one workgroup per CU: more slices buy no speed in the GEMM at
+  // 24,576 rows and cost reduction traffic), within max_slices.
+  int target = c ? c->splitk_target : 256;
+  if (tiles >= target || K <= kUnslicedK) return 1;
+  // Tiles narrower than 128 columns (the odd-width input layers, launched
+  // alone) whose slices would run past 16 k-tiles aim at two workgroups
+  // per CU (the trainer actor's 256 x 288 input layer: 59.0 -> 46.8 us;
+  // the critic's 512 x 64, 12 k-tiles per slice, stays: 24.5 us).
+  if (g.bn < 128 && cdiv(kt, cdiv(target, tiles)) > 16) target *= 2;
+  const int many = whole(std::min(cdiv(target, tiles), max_slices(kt)));
+  if (!apart) return many;
+  const int few = kt < 16 ? 1 : whole(std::min(cdiv(target, tiles), std::max(1LL, kt / 8)));
+  return apart_us(g, M, N, K, few) < apart_us(g, M, N, K, many) ? few : many;
+}
 
 int pick_gemm(const zl_ctx* c, int M, int N, int K, bool a_kc, bool b_kc, bool vec, int epi,
-              bool vec_b, bool kvec, bool fp32_only) {
+              bool vec_b, bool kvec, bool fp32_only, bool apart) {
   const int fp32 = pick_fp32(c, M, N, K, a_kc, b_kc, vec, epi, vec_b);
   const int lay = layout_of(a_kc, b_kc);
   if (fp32_only || (c && c->force_gemm[lay] >= 0) || fp32 < 0) return fp32;
@@ -233,7 +292,12 @@ int pick_gemm(const zl_ctx* c, int M, int N, int K, bool a_kc, bool b_kc, bool v
   const GemmKernel& g = kGemmTable[fp32 - K_GEMM_BASE];
   if (g.kind != G_TILED || strstr(g.name, "xk128")) return fp32;
   const int split = pick_split(c, M, N, K, lay, epi, vec, kvec);
-  return split >= 0 ? split : fp32;
+  if (split < 0) return fp32;
+  if (apart && epi == zk::kEpiStore) {
+    auto us = [&](const GemmKernel& k) { return apart_us(k, M, N, K, slices_of(c, k, M, N, K, epi, true)); };
+    if (us(kGemmTable[split - K_GEMM_BASE]) >= us(g)) return fp32;
+  }
+  return split;
 }
 
 static int pick_fp32(const zl_ctx* c, int M, int N, int K, bool a_kc, bool b_kc, bool vec, int epi,
@@ -375,32 +439,7 @@ static int narrow_rows_per_slice(const zl_ctx* c, int N, int K, int epi) {
 }
 
 int gemm_splits(const zl_ctx* c, int M, int N, int K, bool a_kc, bool b_kc, int epi, bool vec) {
-  const GemmKernel& g = kGemmTable[pick_gemm(c, M, N, K, a_kc, b_kc, vec) - K_GEMM_BASE];
-  if (g.kind == G_NARROW_M) return (int)cdiv(std::max(K, 1), narrow_rows_per_slice(c, N, K, epi));
-  if (!is_tiled(g.kind)) return 1;
-  if (epi != zk::kEpiStore) return 1;
-  const long long tiles = cdiv(M, g.bm) * cdiv(N, g.bn);
-  const long long kt = cdiv(K, g.bk);
-  long long s;
-  if (c && c->force_splits > 0) {
-    s = c->force_splits;
-  } else {
-    // Deep-K, few-tile shapes (the weight gradients, K = batch rows) would
-    // leave most CUs idle: slice K so the grid reaches the split-K target
-    // (256 = one workgroup per CU: more slices buy no speed in the GEMM at
-    // 24,576 rows and cost reduction traffic), within max_slices.
-    int target = c ? c->splitk_target : 256;
-    if (tiles >= target || K <= kUnslicedK) return 1;
-    // Tiles narrower than 128 columns (the odd-width input layers, launched
-    // alone) whose slices would run past 16 k-tiles aim at two workgroups
-    // per CU (the trainer actor's 256 x 288 input layer: 59.0 -> 46.8 us;
-    // the critic's 512 x 64, 12 k-tiles per slice, stays: 24.5 us).
-    if (g.bn < 128 && cdiv(kt, cdiv(target, tiles)) > 16) target *= 2;
-    s = std::min(cdiv(target, tiles), max_slices(kt));
-  }
-  s = std::max<long long>(1, std::min(s, kt));
-  const long long per = cdiv(kt, s);
-  return (int)cdiv(kt, per);
+  return slices_of(c, kGemmTable[pick_gemm(c, M, N, K, a_kc, b_kc, vec) - K_GEMM_BASE], M, N, K, epi, false);
 }
 
 // An upper bound of the split-K scratch over every batch of up to K rows: the
@@ -471,7 +510,7 @@ static zl_status plan_gemm(zl_ctx* c, const GemmDesc& d, GemmPlan& P) {
   P.vec = va && vb;
   const bool plain = !d.rowsum_out && !d.permA && !d.permB && d.splits <= 1;
   const bool kvec = (!d.a_kc || va) && (!d.b_kc || vb);
-  P.kid = pick_gemm(c, d.M, d.N, d.K, d.a_kc, d.b_kc, P.vec, d.epi, vb && plain, kvec, d.fp32);
+  P.kid = pick_gemm(c, d.M, d.N, d.K, d.a_kc, d.b_kc, P.vec, d.epi, vb && plain, kvec, d.fp32, !d.seg_out);
   if (P.kid < 0) return fail(c, ZL_ERR_INVALID, "no GEMM variant for this layout");
   const GemmKernel& g = kGemmTable[P.kid - K_GEMM_BASE];
   const bool vec_ok = g.kind == G_SPLIT ? kvec : P.vec;
@@ -495,7 +534,7 @@ static zl_status plan_gemm(zl_ctx* c, const GemmDesc& d, GemmPlan& P) {
     P.gx = (unsigned)P.splits;
     P.gy = (unsigned)cdiv(d.N, kNarrowCols);
   } else {
-    int splits = d.splits > 0 ? d.splits : gemm_splits(c, d.M, d.N, d.K, d.a_kc, d.b_kc, d.epi, P.vec);
+    int splits = d.splits > 0 ? d.splits : slices_of(c, g, d.M, d.N, d.K, d.epi, !d.seg_out);
     if (d.epi != zk::kEpiStore) splits = 1;
     const long long kt = cdiv(std::max(d.K, 0), g.bk);
     P.per = (int)std::max<long long>(1, cdiv(kt, splits));
