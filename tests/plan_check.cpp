@@ -4,6 +4,8 @@
 //
 //   plan M N K a_kc b_kc epi lda ldb permA permB   "<kernel> <slices>" or "refused"
 //   apart (the same)                                of a product whose partials a launch of its own sums
+//   beside (the same)                               of a layer's gradients that are to share a launch
+//   pair (the same)                                 of one of two such problems in a launch
 //   names                                           every kernel's name on one line
 //   scratch M N K                                   "<floats reserved for up to K rows> <most that any takes>"
 #include "../zealot_amd/csrc/runtime/runtime.cpp"
@@ -19,7 +21,7 @@ void noalloc_release(zl_ctx*) {}
 using namespace zl;
 
 static zl_status plan(zl_ctx& c, int M, int N, int K, bool a_kc, bool b_kc, int epi, int lda, int ldb, bool pa, bool pb,
-                      bool apart, GemmPlan& P) {
+                      const std::string& how, GemmPlan& P) {
   alignas(16) static float mem[4];
   static int perm[4];
   GemmDesc d;
@@ -37,8 +39,9 @@ static zl_status plan(zl_ctx& c, int M, int N, int K, bool a_kc, bool b_kc, int 
   d.permA = pa ? perm : nullptr;
   d.permB = pb ? perm : nullptr;
   zk::ReduceSeg seg;
-  d.seg_out = apart ? nullptr : &seg;
-  return plan_gemm(&c, d, P);
+  d.seg_out = how == "apart" ? nullptr : &seg;
+  d.beside = how == "beside";
+  return plan_gemm(&c, d, P, how == "pair" ? 2 * cdiv(M, 128) * cdiv(N, 128) : 0);
 }
 
 int main() {
@@ -47,11 +50,11 @@ int main() {
   while (std::getline(std::cin, line)) {
     std::istringstream in(line);
     in >> cmd;
-    if (cmd == "plan" || cmd == "apart") {
+    if (cmd == "plan" || cmd == "apart" || cmd == "beside" || cmd == "pair") {
       int M, N, K, a, b, epi, lda, ldb, pa, pb;
       in >> M >> N >> K >> a >> b >> epi >> lda >> ldb >> pa >> pb;
       GemmPlan P;
-      if (plan(c, M, N, K, a, b, epi, lda, ldb, pa, pb, cmd == "apart", P))
+      if (plan(c, M, N, K, a, b, epi, lda, ldb, pa, pb, cmd, P))
         std::puts("refused");
       else
         std::printf("%s %d\n", kGemmTable[P.kid - K_GEMM_BASE].name, P.splits);
@@ -63,11 +66,12 @@ int main() {
       in >> M >> N >> K;
       size_t most = 0;
       for (int k = 1; k <= K; ++k)
-        for (int form = 0; form < 4; ++form) {
+        for (int form = 0; form < 6; ++form) {
+          static const char* const how[3] = {"plan", "apart", "beside"};
           GemmPlan P;
           const int pad = form & 1;  // rows that are not float4-aligned
           if (plan(c, M, N, k, false, false, zk::kEpiStore, (int)round_up(M, 4) + pad, (int)round_up(N, 4) + pad, false,
-                   false, form & 2, P))
+                   false, how[form / 2], P))
             continue;
           if (P.splits > 1) most = std::max(most, (size_t)P.splits * M * N + (size_t)P.splits * M);
         }

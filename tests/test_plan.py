@@ -60,8 +60,8 @@ def test_split_k_scratch_covers_every_shorter_batch(ask, m, n):
 def test_backward_of_a_layer_is_one_launch(ask, rows, n, k):
     """run_gemm_bwd merges a layer's weight and data gradients where both take
     the three-piece variants."""
-    got = ask(("plan", rows, n, k, True, False, ELU_GRAD, k, n, False, False),
-              ("plan", k, n, rows, False, False, STORE, k, n, False, False))
+    got = ask(("beside", rows, n, k, True, False, ELU_GRAD, k, n, False, False),
+              ("beside", k, n, rows, False, False, STORE, k, n, False, False))
     assert [x.split()[0] for x in got] == ["zk_split_ak_bn_dg", "zk_split_am_bn"]
 
 
@@ -97,6 +97,28 @@ def test_products_summed_apart(ask, m, n, k, a, b, want):
     first three measured 10.2, 10.6 and 15.1 us, 15.4, 20.1 and 25.7 as a minibatch
     runs them.)"""
     assert ask(("apart", m, n, k, a, b, STORE, k if a else m, k if b else n, False, False)) == [want]
+
+
+@pytest.mark.parametrize("how,m,n,k,ld,want", [("plan", 4096, 256, 512, 512, False), ("plan", 16_384, 128, 128, 128, False),
+                                               ("plan", 10_000, 256, 512, 512, True), ("pair", 4096, 256, 512, 512, False),
+                                               ("pair", 4608, 256, 512, 512, True), ("plan", 4096, 256, 123, 123, True),
+                                               ("plan", 12_288, 512, 64, 64, True), ("pair", 2048, 512, 512, 512, False)])
+def test_forwards_on_three_pieces(ask, how, m, n, k, ld, want):
+    """By the tiles of the launch: 144 with float4-aligned rows, 64 without."""
+    got = ask((how, m, n, k, True, True, BIAS_N, ld, ld, False, False))[0]
+    assert got.startswith("zk_split_ak_bk") == want, got
+
+
+@pytest.mark.parametrize("how,m,n,k,want", [
+    ("plan", 1000, 512, 512, False), ("plan", 3000, 512, 256, False), ("plan", 4096, 128, 128, True),
+    ("plan", 24_576, 512, 128, True), ("plan", 24_576, 512, 100, False), ("plan", 24_576, 192, 128, False),
+    ("plan", 24_576, 64, 128, False), ("plan", 24_576, 384, 200, False), ("plan", 24_576, 192, 256, True),
+    ("beside", 12_288, 100, 100, False), ("beside", 24_576, 100, 100, True), ("beside", 24_576, 64, 48, False)])
+def test_data_gradients_on_three_pieces(ask, how, m, n, k, want):
+    """Alone in their launch: whole column tiles and k-tiles from 4,096 rows on,
+    others from K = 256 and 192 tiles; beside their weight gradient from 192."""
+    got = ask((how, m, n, k, True, False, ELU_GRAD, (k + 3) // 4 * 4, n, False, False))[0]
+    assert got.startswith("zk_split_ak_bn_dg") == want, got
 
 
 def test_bench_counts_every_gemm_kernel(ask):

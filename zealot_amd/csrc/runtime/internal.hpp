@@ -156,7 +156,7 @@ struct zl_ctx {
   // layout (ZL_GEMM_AKBK / _AKBN / _AMBN / _AMBK), split-K slice count
   // (ZL_SPLITK) and the split-K target grid size (ZL_SPLITK_TARGET).
   int force_gemm[4] = {-1, -1, -1, -1};
-  // Three-piece bf16 GEMMs where pick_gemm's rule takes them (ZL_SPLIT_GEMM=0
+  // Three-piece bf16 GEMMs where pick_split's rule takes them (ZL_SPLIT_GEMM=0
   // turns them off).
   bool split_gemm = true;
   int force_splits = 0;
@@ -247,6 +247,7 @@ struct GemmDesc {
   int ldy = 0;
   float* rowsum_out = nullptr;  // row sums of A (bias gradient of a wgrad)
   int splits = 0;               // 0: heuristic; only kEpiStore may split
+  bool beside = false;          // set by run_gemm_bwd: a layer's gradients that may share a launch
   bool fp32 = false;            // the fp32 MFMA kernels, also where three-piece ones would be faster
   const int* guard = nullptr;
   float* ws = nullptr;          // split-K scratch (floats); nullptr: context scratch
@@ -254,19 +255,7 @@ struct GemmDesc {
   zk::ReduceSeg* seg_out = nullptr;  // set: no reduce launch, describe it here instead
 };
 
-// Variant choice and split-K decision shared by run_gemm and the scratch
-// sizing of composites.
-// vec: both operands can be read as aligned float4 rows (see run_gemm).
-// vec_b: B alone can be read as float4 rows and the problem has no split-K,
-// row sums or gathers (the small-K variants may then take it).
-// kvec: every K-contiguous operand can be read as float4 rows (the three-piece
-// variants read the others by elements). fp32_only: no three-piece variant.
-// apart: split-K partials are summed by a launch of their own.
-int pick_gemm(const zl_ctx* c, int M, int N, int K, bool a_kc, bool b_kc, bool vec = true,
-              int epi = zk::kEpiStore, bool vec_b = false, bool kvec = true, bool fp32_only = false,
-              bool apart = false);
-int gemm_splits(const zl_ctx* c, int M, int N, int K, bool a_kc, bool b_kc, int epi,
-                bool vec = true);
+// Split-K scratch, in floats, of a product over every reduction of up to K.
 size_t gemm_ws_floats(const zl_ctx* c, int M, int N, int K, bool a_kc, bool b_kc, int epi);
 zl_status run_gemm(zl_ctx* c, const GemmDesc& d);
 // One launch for n (1 or 2) problems that pick the same variant (else n
@@ -276,7 +265,9 @@ zl_status run_gemm_batch(zl_ctx* c, const GemmDesc* d, int n);
 // batch d (nd may be 0), as one zk_split_bwd launch when both are single
 // launches of the three-piece variants, else as run_gemm_batch(w) then
 // run_gemm_batch(d).
-zl_status run_gemm_bwd(zl_ctx* c, const GemmDesc* w, int nw, const GemmDesc* d, int nd);
+zl_status run_gemm_bwd(zl_ctx* c, GemmDesc* w, int nw, GemmDesc* d, int nd);
+// Split-K slices that run_gemm_bwd's launch gives a weight gradient.
+zl_status beside_splits(zl_ctx* c, GemmDesc d, int* splits);
 // Block layout of zk_reduce_all over `segs` (fills lanes / blk0 / nqb / nrb);
 // returns the block count (= number of sum-of-squares partials).
 int reduce_all_layout(zk::ReduceSeg* segs, int nseg);

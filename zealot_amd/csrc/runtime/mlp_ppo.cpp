@@ -345,9 +345,12 @@ static zl_status pair_backward(zl_ctx* c, const NetView v[2], const float* param
       if (div == 0) div = dg_tiles >= 6LL * c->cu_count ? 2 : 1;
       if (div > 1)
         for (int j = 0; j < nw; ++j)
-          if (w[j].M > 0 && L[j] - 1 - depth > 0)  // a layer with a data gradient
-            w[j].splits = std::max(1, gemm_splits(c, w[j].M, w[j].N, w[j].K, w[j].a_kc, w[j].b_kc,
-                                                  w[j].epi) / div);
+          if (w[j].M > 0 && L[j] - 1 - depth > 0) {  // a layer with a data gradient
+            int splits = 1;
+            zl_status s = beside_splits(c, w[j], &splits);
+            if (s) return s;
+            w[j].splits = std::max(1, splits / div);
+          }
     }
     zl_status s = ZL_OK;
     if (paired) {

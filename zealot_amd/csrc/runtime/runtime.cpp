@@ -180,42 +180,72 @@ static bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
 constexpr int kUnslicedK = 128;
 inline long long max_slices(long long kt) { return std::max({1LL, kt / 8, std::min(kt / 2, 64LL)}); }
 
+// What the variant choice needs to know beside a problem's sizes, layout and
+// epilogue.
+struct PickTraits {
+  bool vec = true;      // both operands can be read as aligned float4 rows (see plan_gemm)
+  bool vec_b = false;   // B alone can, and no split-K, row sums or gathers (small-K variants)
+  bool kvec = true;     // every K-contiguous operand can (three-piece variants)
+  bool vec_out = true;  // the rows of C and of the ELU' operand are float4-aligned
+  bool fp32 = false;    // no three-piece variant
+  bool apart = false;   // split-K partials are summed by a launch of their own
+  bool beside = false;  // a layer's weight and data gradients, to share a launch
+  long long tiles = 0;  // 128 x 128 tiles of the whole launch (0: of this problem alone)
+};
+
 // The three-piece bf16 variant (gemm_split.hip) of a product, or -1 where the
 // fp32 tiles stay. Its 128 x 128 tiles pay once enough of them are in flight;
 // fewer are bound by one block's serial chain (2 us per k-tile), which the
-// smaller fp32 tiles shorten. Launches of an actor + critic pair, us, fp32 vs
-// three-piece: forward 2,000 x 512 x 128 13 / 16, 2,000 x 512 x 64 9 / 13, 3,000 x 256 x 512 29 / 34,
-// 4,500 x 256 x 512 37 / 33, 24,576 x 256 x 512 108 / 79, 24,576 x 512 x 128
-// 70 / 49; a layer's backward 1,000 x 512 x 256 43 / 28 + 26, 2,000 51 / 33,
-// 24,576 222 / 151; input-layer weight gradient 512 x 128 x 24,576 63 / 48.
-// Feature-major products (L_AK_BN without ELU'), one problem: 128 x 24,576 x
-// 256 26 / 29, 256 x 24,576 x 512 75 / 60. Narrow or half-empty tiles keep fp32.
-// vec, kvec: as in pick_gemm.
-static int pick_split(const zl_ctx* c, int M, int N, int K, int lay, int epi, bool vec, bool kvec) {
+// smaller fp32 tiles shorten. fp32 time over three-piece time, by tiles of the
+// launch:
+// - Forwards: K = 64 to 512 0.6 to 0.9 at 64 to 128, 1.02 to 1.12 at 158, 1.15 at
+//   256, 1.4 at 384; K <= 64 1.03 to 1.06 at 192. Operands that are not float4-
+//   aligned 1.14 to 1.2 from 64 on. (A pair of 3,000 x 256 x 512, 96 tiles, 29 / 34
+//   us, of 4,500 x 256 x 512, 144 tiles, 37 / 33.)
+// - Data gradients in whole tiles and k-tiles, which take the staged epilogue: 0.6
+//   to 1.05 up to 96 tiles below 4,096 rows, 1.05 to 1.6 from there on (the fp32
+//   tiles are 128 wide there); in one launch with the layer's weight gradient 1.03
+//   at 24 (us per minibatch of 48-128-128-8 nets, 42 tiles: 75, apart 87; of
+//   64-256-128-64-12 nets, 24 tiles: 102 / 109, 16 tiles: 98 / 95). Others 0.4 to
+//   0.9, with K >= 256 1.08 to 1.9 from 192 tiles on, unaligned 1.17 to 2 from 288;
+//   beside their weight gradient from 192 tiles on (100 x 100 layers of 24,576 rows
+//   44 us, 63 apart on fp32).
+// - Weight gradients: up to 128 x 128 0.6 to 0.95, 128 x 288 and 128 x 512 0.8 to
+//   0.98 up to 6,000 rows and 1.1 to 1.6 from 10,000, wider 1.02 to 1.2.
+// - Feature-major layers (L_AK_BN), by K where the fp32 tiles read float4 rows (fp32 /
+//   three-piece, us, 256 tiles and 384): 36 13.2 / 17.7, 19.0 / 20.1; 64 13.2 / 17.2,
+//   20.3 / 19.8; 128 19.3 / 20.6, 27.5 / 25.1; 256 28.3 / 27.9, 39.4 / 35.4 (34.0 /
+//   34.7 at 316 tiles).
+// Plain products that are summed apart are weighed by apart_us on top of this.
+static int pick_split(const zl_ctx* c, int M, int N, int K, int lay, int epi, const PickTraits& t) {
   if (!c || !c->split_gemm || lay == L_AM_BK) return -1;
   const long long tiles = cdiv(M, 128) * cdiv(N, 128);
   if (2LL * M * N < tiles * 128 * 128) return -1;
-  // Split-K slices count as blocks.
-  const long long slices =
-      epi == zk::kEpiStore ? std::min(cdiv(256, tiles), max_slices(K / 32)) : 1;
-  long long least = 48;
-  if (lay == L_AK_BK && epi != zk::kEpiStore) least = M <= 2048 ? LLONG_MAX : K <= 64 ? 192 : 64;
-  // Data gradients share a launch with their layer's weight gradient where both
-  // are three-piece (us per minibatch of 48-128-128-8 nets, 42 tiles: 75, apart 87;
-  // of 64-256-128-64-12 nets, 24 tiles: 102 / 109, 16 tiles: 98 / 95).
-  // Feature-major layers, by K where the fp32 tiles read float4 rows
-  // (fp32 / three-piece, us, 256 tiles and 384): 36 13.2 / 17.7, 19.0 / 20.1; 64
-  // 13.2 / 17.2, 20.3 / 19.8; 128 19.3 / 20.6, 27.5 / 25.1; 256 28.3 / 27.9, 39.4 /
-  // 35.4 (34.0 / 34.7 at 316 tiles).
-  if (lay == L_AK_BN)
-    least = epi == zk::kEpiEluGrad ? 24 : epi == zk::kEpiStore || !vec || K > 256 ? 256 : K < 64 ? 512 : 384;
-  if (tiles * slices < least) return -1;
+  const bool half = 2LL * M * N == tiles * 128 * 128;
+  const long long all = std::max(tiles, t.tiles);
+  if (epi == zk::kEpiStore) {
+    const bool weight = lay == L_AM_BN && !t.apart && !t.beside;
+    if (weight && t.vec && (half || tiles == 1)) return -1;
+    if (weight && t.vec && M <= 128 && K < 10000) return -1;
+    // Split-K slices count as blocks.
+    if (tiles * std::min(cdiv(256, tiles), max_slices(K / 32)) < (lay == L_AK_BN ? 256 : 48)) return -1;
+  } else if (lay == L_AK_BK) {
+    if (M <= 2048 || half || all < (K <= 64 ? 192 : t.kvec ? 144 : 64)) return -1;
+  } else if (epi == zk::kEpiEluGrad) {
+    if (N % 128 == 0 && K % 32 == 0 && t.vec_out) {
+      if (t.beside ? tiles < 24 : M < 4096 && all < 128) return -1;
+    } else if (t.beside ? tiles < 192 || half : N <= 128 || tiles < (t.vec ? 192 : 288) || (t.vec && K < 256)) {
+      return -1;
+    }
+  } else if (tiles < (!t.vec || K > 256 ? 256 : K < 64 ? 512 : 384)) {
+    return -1;
+  }
   switch (lay) {
     case L_AK_BK:
-      if (!kvec) return gemm_id("zk_split_ak_bk_s");
+      if (!t.kvec) return gemm_id("zk_split_ak_bk_s");
       return gemm_id(epi != zk::kEpiStore && K > 128 ? "zk_split_ak_bk_acc2" : "zk_split_ak_bk");
     case L_AK_BN:
-      if (!kvec) return gemm_id("zk_split_ak_bn_s");
+      if (!t.kvec) return gemm_id("zk_split_ak_bn_s");
       return gemm_id(epi == zk::kEpiEluGrad ? "zk_split_ak_bn_dg" : "zk_split_ak_bn");
     default:
       return gemm_id("zk_split_am_bn");
@@ -283,17 +313,16 @@ static int slices_of(const zl_ctx* c, const GemmKernel& g, int M, int N, int K, 
   return apart_us(g, M, N, K, few) < apart_us(g, M, N, K, many) ? few : many;
 }
 
-int pick_gemm(const zl_ctx* c, int M, int N, int K, bool a_kc, bool b_kc, bool vec, int epi,
-              bool vec_b, bool kvec, bool fp32_only, bool apart) {
-  const int fp32 = pick_fp32(c, M, N, K, a_kc, b_kc, vec, epi, vec_b);
+static int pick_gemm(const zl_ctx* c, int M, int N, int K, bool a_kc, bool b_kc, int epi, const PickTraits& t) {
+  const int fp32 = pick_fp32(c, M, N, K, a_kc, b_kc, t.vec, epi, t.vec_b);
   const int lay = layout_of(a_kc, b_kc);
-  if (fp32_only || (c && c->force_gemm[lay] >= 0) || fp32 < 0) return fp32;
+  if (t.fp32 || (c && c->force_gemm[lay] >= 0) || fp32 < 0) return fp32;
   // Narrow and small-K shapes keep their own kernels.
   const GemmKernel& g = kGemmTable[fp32 - K_GEMM_BASE];
   if (g.kind != G_TILED || strstr(g.name, "xk128")) return fp32;
-  const int split = pick_split(c, M, N, K, lay, epi, vec, kvec);
+  const int split = pick_split(c, M, N, K, lay, epi, t);
   if (split < 0) return fp32;
-  if (apart && epi == zk::kEpiStore) {
+  if (t.apart && epi == zk::kEpiStore) {
     auto us = [&](const GemmKernel& k) { return apart_us(k, M, N, K, slices_of(c, k, M, N, K, epi, true)); };
     if (us(kGemmTable[split - K_GEMM_BASE]) >= us(g)) return fp32;
   }
@@ -438,10 +467,6 @@ static int narrow_rows_per_slice(const zl_ctx* c, int N, int K, int epi) {
   return (int)std::min(r, full);
 }
 
-int gemm_splits(const zl_ctx* c, int M, int N, int K, bool a_kc, bool b_kc, int epi, bool vec) {
-  return slices_of(c, kGemmTable[pick_gemm(c, M, N, K, a_kc, b_kc, vec) - K_GEMM_BASE], M, N, K, epi, false);
-}
-
 // An upper bound of the split-K scratch over every batch of up to K rows: the
 // slice count is not monotonic in K (slices are whole k-tiles), and a smaller
 // K can take another variant, so each variant's slice limit counts.
@@ -465,8 +490,7 @@ size_t gemm_ws_floats(const zl_ctx* c, int M, int N, int K, bool a_kc, bool b_kc
       s = std::max(s, std::min(cdiv(target, cdiv(M, g.bm) * cdiv(N, g.bn)), max_slices(kt)));
     }
   };
-  const int split = pick_split(c, M, N, K, lay, epi, false, true);  // the form with the lower threshold
-  if (split >= 0) limit(split);
+  if (c && c->split_gemm && lay == L_AM_BN) limit(gemm_id("zk_split_am_bn"));
   for (bool vec : {true, false}) limit(pick_fp32(c, M, N, K, a_kc, b_kc, vec, epi, false));
   return s <= 1 ? 0 : (size_t)s * M * N + (size_t)s * M;
 }
@@ -501,7 +525,8 @@ static bool gathers(const GemmKernel& g, const GemmDesc& d) {
   }
 }
 
-static zl_status plan_gemm(zl_ctx* c, const GemmDesc& d, GemmPlan& P) {
+// launch_tiles: 128 x 128 tiles of all problems of the launch (0: of this one).
+static zl_status plan_gemm(zl_ctx* c, const GemmDesc& d, GemmPlan& P, long long launch_tiles = 0) {
   // float4 row loads need 16-byte aligned rows that cover the padded extent.
   const int a_ext = d.a_kc ? d.K : d.M;
   const int b_ext = d.b_kc ? d.K : d.N;
@@ -510,7 +535,20 @@ static zl_status plan_gemm(zl_ctx* c, const GemmDesc& d, GemmPlan& P) {
   P.vec = va && vb;
   const bool plain = !d.rowsum_out && !d.permA && !d.permB && d.splits <= 1;
   const bool kvec = (!d.a_kc || va) && (!d.b_kc || vb);
-  P.kid = pick_gemm(c, d.M, d.N, d.K, d.a_kc, d.b_kc, P.vec, d.epi, vb && plain, kvec, d.fp32, !d.seg_out);
+  // Rows that the exact-fit forms and the staged epilogue store, and read the
+  // ELU' operand from, as float4 segments.
+  const bool c_vec = aligned16(d.C) && d.ldc % 4 == 0;
+  const bool y_vec = d.epi != zk::kEpiEluGrad || (aligned16(d.Y) && d.ldy % 4 == 0);
+  PickTraits t;
+  t.vec = P.vec;
+  t.vec_b = vb && plain;
+  t.kvec = kvec;
+  t.vec_out = c_vec && y_vec;
+  t.fp32 = d.fp32;
+  t.apart = !d.seg_out;
+  t.beside = d.beside;
+  t.tiles = launch_tiles;
+  P.kid = pick_gemm(c, d.M, d.N, d.K, d.a_kc, d.b_kc, d.epi, t);
   if (P.kid < 0) return fail(c, ZL_ERR_INVALID, "no GEMM variant for this layout");
   const GemmKernel& g = kGemmTable[P.kid - K_GEMM_BASE];
   const bool vec_ok = g.kind == G_SPLIT ? kvec : P.vec;
@@ -541,13 +579,9 @@ static zl_status plan_gemm(zl_ctx* c, const GemmDesc& d, GemmPlan& P) {
     P.splits = (int)std::max<long long>(1, cdiv(kt, P.per));
     P.gx = (unsigned)cdiv(d.M, g.bm);
     P.gy = (unsigned)cdiv(d.N, g.bn);
-    // Every tile and k-tile full: the exact-fit form of the same variant
-    // (which may store C and read the ELU' operand as float4 row segments:
-    // those rows must be 16-byte aligned, unless C is the split-K scratch).
-    const bool c_vec = P.splits > 1 || (aligned16(d.C) && d.ldc % 4 == 0);
-    const bool y_vec = d.epi != zk::kEpiEluGrad || (aligned16(d.Y) && d.ldy % 4 == 0);
-    P.vec_out = c_vec && y_vec;
-    if (d.K > 0 && d.M % g.bm == 0 && d.N % g.bn == 0 && d.K % g.bk == 0 && c_vec && y_vec) {
+    // Every tile and k-tile full: the exact-fit form of the same variant.
+    P.vec_out = (P.splits > 1 || c_vec) && y_vec;  // the split-K scratch is aligned
+    if (d.K > 0 && d.M % g.bm == 0 && d.N % g.bn == 0 && d.K % g.bk == 0 && P.vec_out) {
       const int x = exact_form(P.kid);
       if (x >= 0) P.kid = x;
     }
@@ -583,8 +617,10 @@ static zl_status plan_batch(zl_ctx* c, const GemmDesc* d, int n, BatchLaunch& L,
   if (nl == 0) return ZL_OK;
   const GemmDesc* const* live = L.live;
   GemmPlan* P = L.P;
+  long long tiles = 0;
+  for (int i = 0; i < nl; ++i) tiles += cdiv(live[i]->M, 128) * cdiv(live[i]->N, 128);
   for (int i = 0; i < nl; ++i) {
-    zl_status s = plan_gemm(c, *live[i], P[i]);
+    zl_status s = plan_gemm(c, *live[i], P[i], tiles);
     if (s) return s;
   }
   // Narrow kernels size one grid for both problems. Those that return on
@@ -749,30 +785,41 @@ static zl_status finish_batch(zl_ctx* c, const BatchLaunch& L) {
   return ZL_OK;
 }
 
+static zl_status launch_batch(zl_ctx* c, const BatchLaunch& L) {
+  c->pending_flops = L.flops;
+  c->pending_shape = {L.live[0]->M, L.live[0]->N, L.live[0]->K, L.P[0].splits};
+  zl_status s = launch(c, L.kid, L.gx, L.gy, L.gz, L.B, 0, L.threads);
+  return s ? s : finish_batch(c, L);
+}
+
 zl_status run_gemm_batch(zl_ctx* c, const GemmDesc* d, int n) {
   BatchLaunch L;
   bool one = false;
   zl_status s = plan_batch(c, d, n, L, one);
   if (s || L.nl == 0) return s;
-  if (!one) {
-    s = run_gemm_batch(c, L.live[0], 1);
-    return s ? s : run_gemm_batch(c, L.live[1], 1);
-  }
-  c->pending_flops = L.flops;
-  c->pending_shape = {L.live[0]->M, L.live[0]->N, L.live[0]->K, L.P[0].splits};
-  s = launch(c, L.kid, L.gx, L.gy, L.gz, L.B, 0, L.threads);
-  return s ? s : finish_batch(c, L);
+  if (one) return launch_batch(c, L);
+  s = run_gemm_batch(c, L.live[0], 1);
+  return s ? s : run_gemm_batch(c, L.live[1], 1);
 }
 
-zl_status run_gemm_bwd(zl_ctx* c, const GemmDesc* w, int nw, const GemmDesc* d, int nd) {
-  if (c->merged_bwd && nd > 0) {
+zl_status run_gemm_bwd(zl_ctx* c, GemmDesc* w, int nw, GemmDesc* d, int nd) {
+  auto beside = [&](bool on) {
+    for (int i = 0; i < nw; ++i) w[i].beside = on;
+    for (int i = 0; i < nd; ++i) d[i].beside = on;
+  };
+  if (nd > 0) {
     BatchLaunch W, D;
     bool ow = false, od = false;
+    beside(true);
     zl_status s = plan_batch(c, w, nw, W, ow);
     if (s) return s;
     if (ow && W.nl > 0 && (s = plan_batch(c, d, nd, D, od))) return s;
     if (ow && od && W.nl > 0 && D.nl > 0 && D.kid == gemm_id("zk_split_ak_bn_dg") &&
         W.kid == gemm_id("zk_split_am_bn")) {
+      if (!c->merged_bwd) {
+        s = launch_batch(c, W);
+        return s ? s : launch_batch(c, D);
+      }
       zk::GemmPair a{};
       a.w = W.B;
       a.d = D.B;
@@ -784,9 +831,19 @@ zl_status run_gemm_bwd(zl_ctx* c, const GemmDesc* w, int nw, const GemmDesc* d, 
       if (!s) s = finish_batch(c, W);
       return s ? s : finish_batch(c, D);
     }
+    beside(false);
   }
   zl_status s = run_gemm_batch(c, w, nw);
   return s || nd == 0 ? s : run_gemm_batch(c, d, nd);
+}
+
+// Slices of a weight gradient that is to share its layer's launch.
+zl_status beside_splits(zl_ctx* c, GemmDesc d, int* splits) {
+  GemmPlan P;
+  d.beside = true;
+  zl_status s = plan_gemm(c, d, P);
+  *splits = P.splits;
+  return s;
 }
 
 zl_status run_gemm(zl_ctx* c, const GemmDesc& d) { return run_gemm_batch(c, &d, 1); }
