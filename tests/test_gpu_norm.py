@@ -192,10 +192,12 @@ def test_bad_arguments_rejected(ctx):
         GpuNormalizer(ctx, 5000)
 
 
-@pytest.mark.parametrize("dim,rows", [(8, 32_768), (9, 32_769), (17, 70_001), (1, 33_000), (4096, 300)])
+@pytest.mark.parametrize("dim,rows", [(8, 32_768), (9, 32_769), (17, 70_001), (1, 33_000), (4096, 300),
+                                      (128, 2048), (129, 2048), (265, 600), (1024, 1500), (1025, 256), (100, 2049), (7, 4097)])
 def test_update_merge_edges(ctx, dim, rows):
     """Around one chunk per run of zk_norm_merge (128 runs of 256 rows), columns
-    around a block's eight, one block and hundreds; two updates in a row, so
+    around a block's eight, one block and hundreds; up to eight chunks in one block
+    where that holds the columns, and nine; two updates in a row, so
     that the second starts from a folded count."""
     x = obs_rows(rows + dim, rows, dim)
     norm = GpuNormalizer(ctx, dim)

@@ -164,20 +164,23 @@ __device__ __forceinline__ void chan_merge(float& n1, float& mean, float& m2, fl
   n1 = tot;
 }
 
-// Fold the chunks into the state. A block takes kNormMergeCols columns, each
-// with kNormMergeRuns threads: thread j merges the j-th contiguous run of chunks
-// in row order, neighbouring runs are merged pairwise, and the column's first
+// Fold the chunks into the state. A block takes kNormMergeThreads / T columns, each
+// with T threads (a power of two, one per chunk up to kNormMergeRuns): thread j
+// merges the j-th contiguous run of chunks in row order, neighbouring runs are merged pairwise, and the column's first
 // thread merges the state with the result. The order is fixed, so the result
 // is the same on every run. What bounds it is the serial chain of merges (two
 // divisions and two loads each): one block with 8 runs per column took 27.4 us
 // for 384 chunks x 123 columns, now 7 us: the chain is
 // three chunks and seven pairwise merges (the whole update, commit and apply of
-// 98,304 rows 61.5 -> 40.9 us).
+// 98,304 rows 61.5 -> 40.9 us). Up to eight chunks keep one block, which draws no
+// ticket: 1,000 rows x 123 15.5 us, x 265 19.8 (17.7 and 21.4 on 128 threads per column
+// whatever the chunks, 16.2 and 18.8 on the former single block).
 // The count is read by every block and written by the last one to arrive
 // (p.ticket, cleared by zk_norm_stats).
 __device__ void norm_merge_body(const NormArgs& p) {
-  constexpr int C = kNormMergeCols, T = kNormMergeRuns;
-  __shared__ float s_n[C * T], s_mean[C * T], s_m2[C * T];
+  constexpr int NT = kNormMergeThreads;
+  __shared__ float s_n[NT], s_mean[NT], s_m2[NT];
+  const int T = 1 << p.merge_shift, C = NT >> p.merge_shift;
   const int t = threadIdx.x, j = t / C;
   const int c = blockIdx.x * C + t % C;
   const int per = (p.nchunks + T - 1) / T;
@@ -218,10 +221,11 @@ __device__ void norm_merge_body(const NormArgs& p) {
     p.state[c] = sm;
     p.state[p.dim + c] = sq;
   }
-  __syncthreads();  // every reader of the count in this block is done with it
+  __syncthreads();  // every reader of the count in this block has it
   if (t == 0) {
-    __threadfence();
-    if (atomicAdd(p.ticket, 1) == (int)gridDim.x - 1) p.state[2 * p.dim] = count_add_ones(count0, p.rows);
+    // The block's reads of the count are complete, and it writes nothing that
+    // another block reads: no write-back of the L2 before the ticket.
+    if (gridDim.x == 1 || atomicAdd(p.ticket, 1) == (int)gridDim.x - 1) p.state[2 * p.dim] = count_add_ones(count0, p.rows);
   }
 }
 
@@ -251,7 +255,7 @@ __device__ void norm_commit_body(const NormArgs& p) {
 extern "C" __global__ __launch_bounds__(256) void zk_norm_set(zk::NormArgs p) { zk::norm_set_body(p); }
 extern "C" __global__ __launch_bounds__(256) void zk_norm_apply(zk::NormArgs p) { zk::norm_apply_body(p); }
 extern "C" __global__ __launch_bounds__(256) void zk_norm_stats(zk::NormArgs p) { zk::norm_stats_body(p); }
-extern "C" __global__ __launch_bounds__(zk::kNormMergeCols * zk::kNormMergeRuns) void zk_norm_merge(zk::NormArgs p) {
+extern "C" __global__ __launch_bounds__(zk::kNormMergeThreads) void zk_norm_merge(zk::NormArgs p) {
   zk::norm_merge_body(p);
 }
 extern "C" __global__ __launch_bounds__(zk::kNormFoldThreads) void zk_norm_commit(zk::NormArgs p) {

@@ -440,8 +440,8 @@ struct PolicyArgs {
 constexpr int kNormMaxDim = 4096;
 constexpr int kNormChunkRows = 256;    // rows per partial-statistics chunk
 constexpr int kNormFoldThreads = 1024;  // zk_norm_commit block
-constexpr int kNormMergeCols = 8;       // zk_norm_merge: columns per block,
-constexpr int kNormMergeRuns = 128;     // threads (runs of chunks) per column; a power of two
+constexpr int kNormMergeThreads = 1024;  // zk_norm_merge block,
+constexpr int kNormMergeRuns = 128;      // its most threads (runs of chunks) per column; a power of two
 struct NormArgs {
   const float* x;   // [rows x ldx]
   float* out;       // zk_norm_apply: [rows x ldo]
@@ -451,6 +451,7 @@ struct NormArgs {
   int* ticket;      // zk_norm_merge: blocks done, 0 before it (zk_norm_stats clears it)
   long long rows;
   int dim, ldx, ldo, nchunks;
+  int merge_shift;     // zk_norm_merge: log2 of the threads per column
   int rows_per_block;  // zk_norm_apply
   int unit_prior;   // zk_norm_set: 1 = Normalizer::new, 0 = empty pending state
 };

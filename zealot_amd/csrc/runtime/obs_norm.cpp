@@ -49,8 +49,13 @@ zl_status zl_norm_update(zl_ctx* c, float* state, int dim, const float* x, int l
   a.ldx = ld;
   a.nchunks = (int)nchunks;
   if ((s = launch(c, K_NORM_STATS, (unsigned)nchunks, (unsigned)cdiv(dim, 64), 1, a))) return s;
-  return launch(c, K_NORM_MERGE, (unsigned)cdiv(dim, zk::kNormMergeCols), 1, 1, a, 0,
-                zk::kNormMergeCols * zk::kNormMergeRuns);
+  // A thread per chunk of a column, but up to 8 chunks in one block where that
+  // holds the columns: it has no ticket to draw.
+  long long most = std::min<long long>(nchunks, zk::kNormMergeRuns);
+  if (nchunks <= 8) most = std::min<long long>(most, std::max(1, zk::kNormMergeThreads / dim));
+  while ((2LL << a.merge_shift) <= most || (nchunks > 8 && (1LL << a.merge_shift) < most)) ++a.merge_shift;
+  return launch(c, K_NORM_MERGE, (unsigned)cdiv(dim, zk::kNormMergeThreads >> a.merge_shift), 1, 1, a, 0,
+                zk::kNormMergeThreads);
 }
 
 zl_status zl_norm_commit(zl_ctx* c, float* state, float* pending, int dim) {
