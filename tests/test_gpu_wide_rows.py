@@ -14,13 +14,14 @@ from zealot_amd.rl import GpuMlp
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("m,n", [(3, 2047), (3, 2048), (1, 8191), (2, 8192), (5, 8193), (2, 24_581), (300, 4096)])
+@pytest.mark.parametrize("m,n", [(3, 2047), (3, 2048), (1, 8191), (2, 8192), (5, 8193), (2, 24_581), (300, 4096),
+                                 (512, 2100), (513, 2100), (600, 8191), (600, 8192)])
 def test_row_sum_exact_on_integers(ctx, m, n):
     """Whole numbers below 2^24 in every partial sum: any order gives the same."""
     x = np.random.default_rng(n).integers(-300, 300, (m, n)).astype(np.float32)
     out, dx = ctx.alloc(m), ctx.to_device(x)
     names = launches(ctx, lambda: ops.row_sum(ctx, out, dx, m, n))
-    assert names == ["zk_row_sum_wide" if n >= 2048 else "zk_row_sum"]
+    assert names == ["zk_row_sum_wide" if n >= 8192 or n >= 2048 and m <= 512 else "zk_row_sum"]
     assert np.array_equal(out.numpy(), x.sum(1, dtype=np.float64).astype(np.float32))
 
 

@@ -1375,10 +1375,12 @@ zl_status zl_row_sum(zl_ctx* c, float* out, const float* x, int m, int n) {
   a.rows = m;
   a.cols = n;
   a.ldx = n;
-  // From eight values per thread of the wide block on; below, both measured the
-  // same (3.5 us at 128 x 2,047 on 256 threads and 2,048 on 1,024), and narrow
-  // rows keep the smaller block.
-  if (n >= 2048) return launch(c, K_ROW_SUM_WIDE, (unsigned)m, 1, 1, a, 0, zk::kRowSumWideThreads);
+  // From eight values per thread of the wide block on, and between two and eight
+  // while the rows are no more than two per CU: below, both measured the same
+  // (3.5 us at 128 x 2,047 on 256 threads and 2,048 on 1,024), and more rows fill
+  // the chip with the smaller block (4,096 x 2,048 6.6 us vs 12.8, 1,500 x 4,096 4.1
+  // vs 6.2, 16,384 x 4,096 52 vs 73; 512 x 4,096 4.4 vs 3.6).
+  if (n >= 8192 || (n >= 2048 && m <= 512)) return launch(c, K_ROW_SUM_WIDE, (unsigned)m, 1, 1, a, 0, zk::kRowSumWideThreads);
   return launch(c, K_ROW_SUM, (unsigned)m, 1, 1, a);
 }
 
