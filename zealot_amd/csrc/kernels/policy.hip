@@ -10,9 +10,11 @@
 // Every value is computed as on the multi-launch path: the normalisation is
 // Normalizer::normalize's expression (ppo.rs:198-205), each layer sums its
 // reduction index in 16-wide chunks with lane group s of MFMA step c on
-// index k0 + 4 s + c (the order of the tiled and narrow GEMM kernels), adds
+// index k0 + 4 s + c (the order of the tiled and narrow fp32 GEMM kernels), adds
 // the bias after the sum and applies ELU to the hidden layers, and the
-// log-probability adds its terms in component order.
+// log-probability adds its terms in component order. Layer launches on fp32
+// kernels (chunks of up to 2,048 rows) give the same bits; those that take the
+// three-piece kernels agree to rounding.
 #pragma once
 #include "common.hip"
 
@@ -37,9 +39,8 @@ __device__ __forceinline__ float4 policy_chunk(const float* Wp, unsigned w, int 
 }
 
 // A wavefront's nu tiles of one layer, src [16 x 16 kc] in LDS times the packed
-// chunks at w[u] (bytes from Wp). Issue the first chunks of every tile, without
-// a branch (a wavefront with no tile re-reads chunks of another's), so that the
-// loads stay in flight over the code between the layers ...
+// chunks at w[u] (bytes from Wp). Issue the first chunks of its tiles, which stay in
+// flight over the code between the layers ...
 __device__ __forceinline__ void policy_prime(float4 (&ring)[kPolicyDepth], const float* Wp, const unsigned (&w)[2], int nu,
                                              int kc) {
 #pragma unroll
@@ -86,10 +87,12 @@ __device__ __forceinline__ void policy_sum(floatx4 (&acc)[2], float4 (&ring)[kPo
 // 0.93 MB of weights (headline actor) arrive one dependent round of loads
 // after another; the fp32 MFMAs alone take 12 us, and 24 us at 4,096 rows (two
 // blocks per CU). The loads therefore run as a ring that is refilled slot by
-// slot, a layer's first chunks and its bias are on their way over the epilogue
-// and the barrier of the layer before, and the input rows and log_std travel
-// with the normaliser's statistics. A step of both headline nets: 28.5 -> 22.9 us
-// at 64 rows, 50.2 -> 40.7 us at 4,096.
+// slot, a layer's first chunks and its bias are on their way over the barrier of
+// the layer before (issued before that layer's epilogue they cost four spilled
+// registers: with the loads of idle wavefronts 4,096 rows of 48-128-128-8 nets 13.4 us,
+// now 11.5), and the input rows and log_std travel with the normaliser's
+// statistics. A step of both headline nets: 28.3 -> 22.0 us at 64 rows, 51 -> 38.3 us
+// at 4,096.
 __device__ void policy_body(const PolicyArgs& p) {
   __shared__ __align__(16) float act[2][kPolicyRows * kPolicyPitch];
   __shared__ float s_mu[kPolicyMaxWidth], s_sd[kPolicyMaxWidth];
@@ -128,7 +131,7 @@ __device__ void policy_body(const PolicyArgs& p) {
 #pragma unroll
     for (int u = 0; u < 2; ++u) bias[u] = bl[(unsigned)min(16 * tile[u] + lr, q.dims[l + 1] - 1)];
     const float* Wp = q.wp + q.wp_off[l];
-    policy_prime(ring, Wp, woff, nu, kc);
+    if (nu > 0) policy_prime(ring, Wp, woff, nu, kc);
   };
   begin_layer(0);
   const bool sampling = blockIdx.y == 0 && p.sample;
@@ -173,25 +176,23 @@ __device__ void policy_body(const PolicyArgs& p) {
     const float* src = act[cur] + lr * kPolicyPitch + 4 * lg;
     float* dst = act[cur ^ 1];
     floatx4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
-    const int mine = nu, n[2] = {16 * tile[0] + lr, 16 * tile[1] + lr};
-    const float b[2] = {bias[0], bias[1]};
-    if (mine == 2)
+    if (nu == 2)
       policy_sum<2>(acc, ring, Wp, woff, kc, src);
-    else if (mine == 1)
+    else if (nu == 1)
       policy_sum<1>(acc, ring, Wp, woff, kc, src);
-    // The next layer's first weights travel during the epilogue and the barrier.
-    if (!last) begin_layer(l + 1);
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
-      if (u >= mine || n[u] >= N) continue;
+      const int n = 16 * tile[u] + lr;
+      if (u >= nu || n >= N) continue;
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int row = 4 * lg + r;
-        const float v = last ? acc[u][r] + b[u] : elu(acc[u][r] + b[u]);
-        dst[row * kPolicyPitch + n[u]] = v;
-        if (last && q.out && row < nr) q.out[(r0 + row) * q.ldo + n[u]] = v;
+        const float v = last ? acc[u][r] + bias[u] : elu(acc[u][r] + bias[u]);
+        dst[row * kPolicyPitch + n] = v;
+        if (last && q.out && row < nr) q.out[(r0 + row) * q.ldo + n] = v;
       }
     }
+    if (!last) begin_layer(l + 1);  // its first weights travel over the barrier
     __syncthreads();
     cur ^= 1;
   }
