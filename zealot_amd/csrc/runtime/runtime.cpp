@@ -349,7 +349,7 @@ static int pick_fp32(const zl_ctx* c, int M, int N, int K, bool a_kc, bool b_kc,
       // 64-512), up to 32 rows while they give a CU one (29 x 4,096 x 512:
       // 6.7 vs 8.5 us on 32-column blocks, 29 x 8,192: 11.8 vs 8.6).
       if (M <= 16) return gemm_id("zk_narrow_f1");
-      if (M <= 32 && N <= 4096) return gemm_id("zk_narrow_f2");
+      if (M <= 32 && cdiv(N, kNarrowFCols) <= 256) return gemm_id("zk_narrow_f2");
       // Rows of A that are aligned but no whole chunks are read by elements
       // here and by float4 on the 64 x 64 tiles: one tile per CU (256 x 1,000 x 264
       // 10.2 vs 13.0 us, 256 x 1,500 16.9 vs 12.8, 512 x 1,000 x 520 29.3 vs 19.8).
