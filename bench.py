@@ -47,7 +47,8 @@ HBM_PEAK = 8.0e12  # bytes/s
 # averaged over an update's launch mix; reported as roofline.traffic for the
 # dominant kernel when it is one of these.
 MEASURED_TRAFFIC = {
-    "zk_gemm_ak_bk_128x128x32_w24_x": 150.3e6,
+    "zk_split_bwd": 353.9e6,
+    "zk_gemm_ak_bk_128x128x32_w24_x": 149.7e6,
 }
 
 

@@ -324,9 +324,10 @@ __device__ __forceinline__ void narrow_m_body(const GemmArgs& p) {
 // C = A . B with few tiles: a block takes 16 MT rows x 16 NT columns of C, its
 // wavefronts contiguous runs of the K chunks (loads of four chunks issued
 // together), and their partials are added in wavefront order from LDS. On 64 x 64
-// tiles such a product is a handful of blocks, each serial over K: 18.1 us for
-// 29 x 4,096 x 512 (64 blocks), now 6.7 (256 blocks, 8.4 MB of B at 1.3 TB/s:
-// a launch, one trip to memory, the fold).
+// tiles such a product is a handful of blocks, each serial over K: 18.1 us per call in
+// a row of calls for 29 x 4,096 x 512 (64 blocks), now 6.7 (256 blocks; a launch by
+// itself, its start and end with it, 9.3 us: 8.4 MB of B at 0.9 TB/s, one trip to
+// memory and the fold).
 // VEC: K % 16 == 0 and A's rows 16-byte aligned.
 template <int MT, int NT, bool VEC>
 __device__ __forceinline__ void narrow_f_body(const GemmArgs& p, float (&red)[kNarrowFWaves][MT * NT][4][64]) {

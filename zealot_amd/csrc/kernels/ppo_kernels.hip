@@ -666,9 +666,10 @@ __device__ void row_sum_body(const RowSumArgs& p) {
 
 // Rows of thousands of values: kRowSumWideThreads per row, eight loads in flight
 // each. One 256-thread block per row with one load per iteration was a chain of
-// cols / 256 trips to memory: 24.7 us for 128 x 24,576 and for 256 x 24,576
-// (12.6 and 25 MB), now
-// 3.6 us (3.4 and 6.7 TB/s, from the last-level cache; 9.2 us for 512 x 24,576).
+// cols / 256 trips to memory: 24.7 us per call for 128 x 24,576, for 256 and for 512
+// (12.6 to 50 MB), now 3.3, 3.6 and 9.2 us in a row of calls (the operand in the
+// last-level cache; a launch by itself, its start and end with it, 6.0 us for 128 rows
+// and 6.4 for 256: 2.1 and 3.9 TB/s).
 // Loads stay dwords, coalesced at any alignment and row stride.
 __device__ void row_sum_wide_body(const RowSumArgs& p) {
   __shared__ float red[kRowSumWideThreads / 64];
