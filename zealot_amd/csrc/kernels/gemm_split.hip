@@ -547,7 +547,7 @@ __device__ __forceinline__ void split_tile(char* __restrict__ smem, const GemmAr
 // Naming: a{k,m} = A K- or M-contiguous, b{k,n} = B K- or N-contiguous, _s
 // element loads of K-contiguous rows that are not 16-byte aligned, _dg the
 // data gradients (ELU' epilogue), _acc2 the forwards with K > 128, whose errors
-// pass through every later layer and the probability ratio.
+// pass through every later layer.
 ZK_SPLIT(zk_split_ak_bk, true, true, true, false, false)
 ZK_SPLIT(zk_split_ak_bk_acc2, true, true, true, false, true)
 ZK_SPLIT(zk_split_ak_bk_s, true, true, false, false, false)
