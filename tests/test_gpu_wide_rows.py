@@ -73,10 +73,10 @@ def test_feature_major_output_layer(ctx, m, n, k):
         assert np.all(np.abs(out.numpy() - ref) <= bound)
 
 
-@pytest.mark.parametrize("rows", [1, 63, 64, 65, 383, 384, 385])
+@pytest.mark.parametrize("rows", [1, 63, 64, 65, 383, 384, 385, 511, 512, 513])
 @pytest.mark.parametrize("dims", [[48, 80, 64, 16], [30, 512, 100, 33, 5]])
 def test_short_batches(ctx, rows, dims):
-    """Forward strips and data gradients of up to 384 rows and the row after,
+    """Forward strips and data gradients of up to 512 rows and the row after,
     widths off the 16 and 32 column tiles; against the oracle with the bar of
     the layer GEMMs (1e-4 of each tensor's largest value)."""
     g = np.random.default_rng(rows)
@@ -89,14 +89,14 @@ def test_short_batches(ctx, rows, dims):
     names = launches(ctx, lambda: mlp.forward(dx, rows))
     # Strips for the layers wider than 32 that read whole chunks of 16.
     wide = [i for i, o in zip(dims, dims[1:]) if o > 32 and i % 16 == 0]
-    if rows <= 384:
+    if rows <= 512:
         assert names.count("zk_narrow_n1_v") >= len(wide), names
     else:
         assert any(x.startswith("zk_gemm_ak_bk") for x in names), names
     ref = zo.mlp_forward(dims, params, x)[-1]
     assert np.abs(mlp.output(rows) - ref).max() <= 1e-4 * np.abs(ref).max()
     names = launches(ctx, lambda: mlp.backward(dg))
-    assert ("zk_narrow_f22" in names) == (rows <= 384 and any(o > 32 for o in dims[2:])), names
+    assert ("zk_narrow_f22" in names) == (rows <= 512 and any(o > 32 for o in dims[2:])), names
     got, (ref, _) = mlp.read_grads(), zo.mlp_backward(dims, params, x, gout)
     o = 0
     for i, j in zip(dims, dims[1:]):

@@ -81,7 +81,12 @@ struct GemmKernel {
 constexpr int kNarrowRows = 64;
 constexpr int kNarrowKCols = 32;
 constexpr int kNarrowCols = 64;
-constexpr int kShortRows = 384;   // rows up to which a minibatch's layers are latency-bound
+// Rows up to which a minibatch's layers are latency-bound and run as strips, K
+// split over wavefronts, the last hidden layer outside zk_head. Per minibatch
+// with it / without, at 400, 512 and 576 rows: 123-512-256-128 nets 118 / 128,
+// 112 / 117, 125 / 121 us; 265-256-256-128 nets 108 / 124, 102 / 112, 114 /
+// 116 us; 48-128-128 nets 62 / 66, 58 / 60, 60 / 63 us.
+constexpr int kShortRows = 512;
 constexpr int kNarrowFCols = 16;  // columns per block of the feature-major forward
 constexpr int kNarrowSliceQuantum = 64;
 

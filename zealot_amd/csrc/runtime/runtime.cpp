@@ -337,7 +337,8 @@ static int pick_fp32(const zl_ctx* c, int M, int N, int K, bool a_kc, bool b_kc,
     const long long tiles = cdiv(M, 32) * cdiv(N, 32);
     if (epi == zk::kEpiEluGrad) {
       // Data gradients of a short minibatch: per minibatch of the headline nets
-      // 4-7 us less than the 64 x 64 tiles at 64-384 rows, 7 us more at 768.
+      // 4-7 us less than the 64 x 64 tiles at 64-384 rows, 7 us more at 768
+      // (the line for all three parts of a short minibatch: kShortRows).
       if (M <= kShortRows && tiles <= 192) return gemm_id("zk_narrow_f22");
     } else {
       // Feature-major layers with few tiles, against the 64 x 64 ones: 29 x
